@@ -27,6 +27,7 @@ namespace {
 
 typedef __bf16 bf16;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
+typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
 int mfail(int code, const char *fmt, ...) {
@@ -63,67 +64,102 @@ struct GemmArgs {
   int ldc, ldt;
 };
 
-constexpr int BM = 64, BN = 64, BK = 32, LDK = BK + 8;
-
-// 256 threads: four waves, each owning a 32 x 32 quarter of the 64 x 64 block
-// tile as 2 x 2 MFMA tiles of 16 x 16.  MFMA 16x16x32 operand layout: lane l
-// holds A[l % 16][8 (l / 16) .. +7] and B[8 (l / 16) .. +7][l % 16] (here B
-// is stored [n][k], so also row l % 16, eight consecutive k); the result
-// D[4 (l / 16) + r][l % 16] is its r-th accumulator.
-template <int EPI>
-__global__ __launch_bounds__(256) void gemm_nt(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) bf16 As[BM][LDK];
-  __shared__ __attribute__((aligned(16))) bf16 Bs[BN][LDK];
+// A workgroup of WM x WN waves, each forming TM x TN MFMA tiles of 16 x 16
+// over the whole of K.  The products here have few rows (a batch), so a
+// launch fills the chip only with small tiles and its time is the latency of
+// the operand loads: each wave reads its operands from global memory straight
+// into registers in MFMA layout, U steps of 32 at a time with the next U
+// steps already in flight; no barrier and no LDS round trip per step.  Every
+// element is one chain of products in ascending k, so its bits do not depend
+// on the tile shape.  The result goes through LDS once, so that the epilogue
+// reads and writes whole lines (16 bytes per lane along the rows, and along
+// the columns for the transpose).
+// MFMA 16x16x32 operand layout: lane l holds A[l % 16][8 (l / 16) .. +7] and
+// B[8 (l / 16) .. +7][l % 16] (B is stored [n][k], so also row l % 16, eight
+// consecutive k); the result D[4 (l / 16) + r][l % 16] is its r-th
+// accumulator.
+template <int EPI, int TM, int TN, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_nt(GemmArgs g) {
+  constexpr int MT = 16 * TM * WM, NT = 16 * TN * WN, THREADS = 64 * WM * WN, U = 16 / (TM + TN);
+  __shared__ __attribute__((aligned(16))) float ct[MT][NT + 4];
+  __shared__ __attribute__((aligned(16))) bf16 tr[NT][MT + 8];  // transposed BF16 result
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  const int lr = tid >> 2, lk = (tid & 3) * 8;  // this thread's 16-byte piece of each operand tile
-  floatx4 acc[2][2];
-  for (int i = 0; i < 2; i++)
-    for (int j = 0; j < 2; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const bf16 *ga = g.A + (long)(m0 + lr) * g.lda + lk;
-  const bf16 *gb = g.B + (long)(n0 + lr) * g.ldb + lk;
-  for (int k0 = 0; k0 < g.K; k0 += BK) {
-    *(uint4 *)&As[lr][lk] = *(const uint4 *)(ga + k0);
-    *(uint4 *)&Bs[lr][lk] = *(const uint4 *)(gb + k0);
-    __syncthreads();
-    bf16x8 a[2], b[2];
-    for (int i = 0; i < 2; i++) a[i] = *(const bf16x8 *)&As[wm + i * 16 + (lane & 15)][8 * (lane >> 4)];
-    for (int j = 0; j < 2; j++) b[j] = *(const bf16x8 *)&Bs[wn + j * 16 + (lane & 15)][8 * (lane >> 4)];
-    for (int i = 0; i < 2; i++)
-      for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
+  const int m0 = blockIdx.y * MT, n0 = blockIdx.x * NT;
+  const int wm = 16 * TM * (wave / WN), wn = 16 * TN * (wave % WN);
+  floatx4 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const bf16 *ga = g.A + (long)(m0 + wm + (lane & 15)) * g.lda + 8 * (lane >> 4);
+  const bf16 *gb = g.B + (long)(n0 + wn + (lane & 15)) * g.ldb + 8 * (lane >> 4);
+  const int ks = g.K / 32;
+  bf16x8 a[2][U][TM], b[2][U][TN];
+  // loads of the steps k .. k + U - 1 (past the end the last step is read
+  // again, and not multiplied)
+  auto load = [&](int slot, int k) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const long o = 32l * min(k + u, ks - 1);
+#pragma unroll
+      for (int i = 0; i < TM; i++) a[slot][u][i] = *(const bf16x8 *)(ga + (long)i * 16 * g.lda + o);
+#pragma unroll
+      for (int j = 0; j < TN; j++) b[slot][u][j] = *(const bf16x8 *)(gb + (long)j * 16 * g.ldb + o);
+    }
+  };
+  auto multiply = [&](int slot, int k) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (k + u < ks) {  // uniform
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int j = 0; j < TN; j++)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[slot][u][i], b[slot][u][j], acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  load(0, 0);
+  for (int k = 0; k < ks; k += 2 * U) {
+    load(1, k + U);
+    multiply(0, k);
+    load(0, k + 2 * U);
+    multiply(1, k + U);
   }
-  for (int i = 0; i < 2; i++) {
-    for (int j = 0; j < 2; j++) {
-      const int n = n0 + wn + j * 16 + (lane & 15);
-      const int mb = m0 + wm + i * 16 + 4 * (lane >> 4);
-      bf16 t4[4];
-      for (int r = 0; r < 4; r++) {
-        const int m = mb + r;
-        const long o = (long)m * g.ldc + n;
-        const float c = acc[i][j][r];
-        if constexpr (EPI == EPI_GELU) {
-          const float z = c + g.bias[n];
-          g.Cf[o] = z;
-          const bf16 h = (bf16)gelu(z);
-          g.Cb[o] = h;
-          t4[r] = h;
-        } else if constexpr (EPI == EPI_LINEAR) {
-          g.Cf[o] = c + g.bias[n];
-        } else if constexpr (EPI == EPI_DGELU) {
-          const bf16 d = (bf16)(c * gelu_grad(g.Zprev[o]));
-          g.Cb[o] = d;
-          t4[r] = d;
-        } else {
-          g.Cf[o] = c;
-        }
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) ct[wm + 16 * i + 4 * (lane >> 4) + r][wn + 16 * j + (lane & 15)] = acc[i][j][r];
+  __syncthreads();
+  for (int q = tid; q < MT * NT / 4; q += THREADS) {
+    const int lm = q / (NT / 4), ln = 4 * (q % (NT / 4));
+    floatx4 c = *(const floatx4 *)&ct[lm][ln];
+    const int n = n0 + ln;
+    const long o = (long)(m0 + lm) * g.ldc + n;
+    if constexpr (EPI == EPI_GELU || EPI == EPI_LINEAR) c += *(const floatx4 *)(g.bias + n);
+    if constexpr (EPI != EPI_DGELU) *(floatx4 *)(g.Cf + o) = c;
+    if constexpr (EPI == EPI_GELU || EPI == EPI_DGELU) {
+      bf16x4 h;
+      if constexpr (EPI == EPI_DGELU) {
+        const floatx4 z = *(const floatx4 *)(g.Zprev + o);
+#pragma unroll
+        for (int r = 0; r < 4; r++) h[r] = (bf16)(c[r] * gelu_grad(z[r]));
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++) h[r] = (bf16)gelu(c[r]);
       }
-      if constexpr (EPI == EPI_GELU || EPI == EPI_DGELU) {
-        // rows mb..mb+3 of column n are consecutive in the transpose
-        bf16 *t = g.Cbt + (long)n * g.ldt + mb;
-        for (int r = 0; r < 4; r++) t[r] = t4[r];
-      }
+      *(bf16x4 *)(g.Cb + o) = h;
+#pragma unroll
+      for (int r = 0; r < 4; r++) tr[ln + r][lm] = h[r];
+    }
+  }
+  if constexpr (EPI == EPI_GELU || EPI == EPI_DGELU) {
+    __syncthreads();
+    for (int q = tid; q < MT * NT / 8; q += THREADS) {
+      const int ln = q / (MT / 8), lm = 8 * (q % (MT / 8));
+      *(bf16x8 *)(g.Cbt + (long)(n0 + ln) * g.ldt + m0 + lm) = *(const bf16x8 *)&tr[ln][lm];
     }
   }
 }
@@ -290,11 +326,21 @@ int malloc_zero(se2w_mlp *m, T **p, size_t n) {
   return SE2W_OK;
 }
 
+// Tile rule: 64 x 64 when that gives every CU a workgroup (256 of them), else
+// 32 x 32 when that does, else 16 x 16 with one wave per workgroup: a smaller
+// tile re-reads the operands more often, a larger one leaves CUs idle.
+constexpr int kCUs = 256;
 template <int EPI>
 int gemm(se2w_mlp *m, const GemmArgs &g) {
-  if (g.M % BM || g.N % BN || g.K % BK || g.lda % 8 || g.ldb % 8)
+  if (g.M % 64 || g.N % 64 || g.K % 32 || g.lda % 8 || g.ldb % 8)
     return mfail(SE2W_ERR_ARG, "product shape %d x %d x %d not tileable", g.M, g.N, g.K);
-  hipLaunchKernelGGL((gemm_nt<EPI>), dim3(g.N / BN, g.M / BM), dim3(256), 0, m->stream, g);
+  const long tiles64 = (long)(g.M / 64) * (g.N / 64);
+  if (tiles64 >= kCUs)
+    hipLaunchKernelGGL((gemm_nt<EPI, 2, 2, 2, 2>), dim3(g.N / 64, g.M / 64), dim3(256), 0, m->stream, g);
+  else if (4 * tiles64 >= kCUs)
+    hipLaunchKernelGGL((gemm_nt<EPI, 1, 1, 2, 2>), dim3(g.N / 32, g.M / 32), dim3(256), 0, m->stream, g);
+  else
+    hipLaunchKernelGGL((gemm_nt<EPI, 1, 1, 1, 1>), dim3(g.N / 16, g.M / 16), dim3(64), 0, m->stream, g);
   return SE2W_OK;
 }
 

@@ -50,7 +50,7 @@ __device__ __forceinline__ float gelu_grad(float z) {
   return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-enum { EPI_GELU = 0, EPI_LINEAR = 1, EPI_DGELU = 2, EPI_STORE = 3 };
+enum { EPI_GELU = 0, EPI_LINEAR = 1, EPI_DGELU = 2 };
 
 struct GemmArgs {
   const bf16 *A;  // [M][lda]
@@ -212,25 +212,17 @@ __global__ void k_sum_parts(const double *part, int n, double inv_count, double 
   }
 }
 
-// Bias gradient: gb[o] = sum over the batch of dZ[b][o] (rows of the transpose).
-__global__ void k_bias_grad(const bf16 *dZt, int B, int N, float *gb) {
-  const int o = blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= N) return;
-  const bf16 *row = dZt + (long)o * B;
-  float s = 0.f;
-  for (int b = 0; b < B; b++) s += (float)row[b];
-  gb[o] = s;
-}
-
 struct AdamArgs {
   float lr, b1, b2, eps, bc1, bc2;  // bc = 1 - beta^t
   float wd;                         // decoupled weight decay (AdamW); 0 = Adam
 };
 
+// The fused multiply-adds are spelled out, so that every kernel that inlines
+// the update rounds alike.
 __device__ __forceinline__ float adam_update(float &w, float &m, float &v, float g, const AdamArgs &a) {
-  m = a.b1 * m + (1.f - a.b1) * g;
-  v = a.b2 * v + (1.f - a.b2) * g * g;
-  w -= a.lr * ((m / a.bc1) / (sqrtf(v / a.bc2) + a.eps) + a.wd * w);
+  m = fmaf(a.b1, m, (1.f - a.b1) * g);
+  v = fmaf(a.b2, v, (1.f - a.b2) * g * g);
+  w = fmaf(-a.lr, fmaf(a.wd, w, (m / a.bc1) / (sqrtf(v / a.bc2) + a.eps)), w);
   return w;
 }
 
@@ -267,6 +259,138 @@ __global__ void k_adam_b(float *b, float *m, float *v, const float *g, int n, Ad
   v[i] = vv;
 }
 
+// One layer of the grouped weight kernel.
+struct WgradLayer {
+  const bf16 *dZt;  // [out][B]     gradient of the pre-activation, transposed
+  const bf16 *Ht;   // [in_pad][B]  the layer's input, transposed
+  int out, in_pad;
+  int tile0;        // its first workgroup; it has (out / 64) (in_pad / 64) tiles, then ceil(out / 256) bias blocks
+  float *W, *mW, *vW, *gW, *b, *mb, *vb, *gb;
+  bf16 *Wb, *Wtb;
+};
+
+// Weight and bias gradients of every layer in one launch, and with ADAM the
+// update in place of storing them: gW = dZt Ht^T (K = the batch) never goes
+// to memory.  The update moves 28 bytes per weight (W, m, v read and written,
+// both BF16 copies written), which bounds the kernel: a workgroup takes a
+// 64 x 64 tile of W, whose product needs only 2 x 64 rows of the batch.  The
+// four waves form a 32 x 32 quarter each from registers (as gemm_nt, one
+// chain per element in ascending k), and the tile goes through LDS so that
+// the update streams whole lines.  The bias blocks sum a row of dZt per
+// thread in ascending order, with eight 16-byte loads in flight.
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_wgrad(const WgradLayer *layers, int nl, int B, AdamArgs a) {
+  __shared__ __attribute__((aligned(16))) float gt[64][68];
+  __shared__ __attribute__((aligned(16))) bf16 tr[64][72];
+  const int tid = threadIdx.x;
+  int l = nl - 1;
+  while (l > 0 && (int)blockIdx.x < layers[l].tile0) l--;
+  const WgradLayer L = layers[l];
+  const int t = blockIdx.x - L.tile0, tx = L.in_pad / 64, nt = tx * (L.out / 64);
+  if (t >= nt) {  // bias block
+    const int o = (t - nt) * 256 + tid;
+    if (o >= L.out) return;
+    const bf16 *row = L.dZt + (long)o * B;
+    float s = 0.f;
+    for (int k = 0; k < B; k += 64) {
+      bf16x8 x[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) x[q] = *(const bf16x8 *)(row + k + 8 * q);
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+#pragma unroll
+        for (int r = 0; r < 8; r++) s += (float)x[q][r];
+    }
+    if constexpr (ADAM) {
+      float w = L.b[o], mm = L.mb[o], vv = L.vb[o];
+      adam_update(w, mm, vv, s, a);
+      L.b[o] = w;
+      L.mb[o] = mm;
+      L.vb[o] = vv;
+    } else {
+      L.gb[o] = s;
+    }
+    return;
+  }
+  const int m0 = 64 * (t / tx), n0 = 64 * (t % tx);
+  const int wave = tid >> 6, lane = tid & 63, wm = 32 * (wave >> 1), wn = 32 * (wave & 1);
+  // this thread's part of the update: rows er + 16 q, four columns from ec
+  const int er = tid >> 4, ec = 4 * (tid & 15);
+  floatx4 w4[4], m4[4], v4[4];
+  if constexpr (ADAM) {  // issued first: their latency overlaps the product
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const long o = (long)(m0 + er + 16 * q) * L.in_pad + n0 + ec;
+      w4[q] = *(const floatx4 *)(L.W + o);
+      m4[q] = *(const floatx4 *)(L.mW + o);
+      v4[q] = *(const floatx4 *)(L.vW + o);
+    }
+  }
+  floatx4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const bf16 *ga = L.dZt + (long)(m0 + wm + (lane & 15)) * B + 8 * (lane >> 4);
+  const bf16 *gb = L.Ht + (long)(n0 + wn + (lane & 15)) * B + 8 * (lane >> 4);
+  for (int k = 0; k < B; k += 64) {  // B is a multiple of 64
+    bf16x8 x[2][2], y[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        x[u][i] = *(const bf16x8 *)(ga + (long)i * 16 * B + k + 32 * u);
+        y[u][i] = *(const bf16x8 *)(gb + (long)i * 16 * B + k + 32 * u);
+      }
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[u][i], y[u][j], acc[i][j], 0, 0, 0);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) gt[wm + 16 * i + 4 * (lane >> 4) + r][wn + 16 * j + (lane & 15)] = acc[i][j][r];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int lm = er + 16 * q;
+    const long o = (long)(m0 + lm) * L.in_pad + n0 + ec;
+    const floatx4 g = *(const floatx4 *)&gt[lm][ec];
+    if constexpr (ADAM) {
+      bf16x4 h;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        float w = w4[q][r], mm = m4[q][r], vv = v4[q][r];
+        adam_update(w, mm, vv, g[r], a);
+        w4[q][r] = w;
+        m4[q][r] = mm;
+        v4[q][r] = vv;
+        h[r] = (bf16)w;
+        tr[ec + r][lm] = h[r];
+      }
+      *(floatx4 *)(L.W + o) = w4[q];
+      *(floatx4 *)(L.mW + o) = m4[q];
+      *(floatx4 *)(L.vW + o) = v4[q];
+      *(bf16x4 *)(L.Wb + o) = h;
+    } else {
+      *(floatx4 *)(L.gW + o) = g;
+    }
+  }
+  if constexpr (ADAM) {
+    __syncthreads();
+    for (int q = tid; q < 64 * 8; q += 256) {
+      const int ln = q >> 3, lm = 8 * (q & 7);
+      *(bf16x8 *)(L.Wtb + (long)(n0 + ln) * L.out + m0 + lm) = *(const bf16x8 *)&tr[ln][lm];
+    }
+  }
+}
+
 // BF16 copies of the FP32 master weights (after set_params / init).
 __global__ void k_to_bf16(const float *W, int rows, int cols, bf16 *Wb, bf16 *Wtb) {
   const long n = (long)rows * cols;
@@ -299,6 +423,8 @@ struct se2w_mlp {
   float *Y = nullptr, *Tb = nullptr;
   float *Xs = nullptr, *Ts = nullptr;  // staging of one host batch
   int *idx = nullptr;                  // batch row indices
+  WgradLayer *wgrad = nullptr;         // [nl] the grouped weight kernel's layers
+  int wgrad_blocks = 0;
   float *X = nullptr, *T = nullptr;    // training data
   int ndata = 0;
   double *part = nullptr, *acc = nullptr;
@@ -375,50 +501,38 @@ int forward(se2w_mlp *m) {
   return SE2W_OK;
 }
 
-// Loss of the batch (added to acc[slot] / count) and all parameter gradients.
+// Loss of the batch (added to acc[slot] / count) and the gradient of every
+// pre-activation.
 int backward(se2w_mlp *m, int slot, double inv_count) {
   MlpLayer &Lo = m->L[m->nl - 1];
   const float scale = 2.0f / ((float)m->B * (float)m->out);
   hipLaunchKernelGGL(k_loss, dim3(m->nparts), dim3(256), 0, m->stream, m->Y, m->Tb, m->B, m->out, scale, Lo.dZ,
                      Lo.dZt, m->part);
   hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(64), 0, m->stream, m->part, m->nparts, inv_count, m->acc, slot);
-  for (int l = m->nl - 1; l >= 0; l--) {
+  for (int l = m->nl - 1; l > 0; l--) {
     MlpLayer &Ly = m->L[l];
-    GemmArgs g = {};
-    g.A = Ly.dZt;
-    g.lda = m->B;
-    g.B = l == 0 ? m->H0t : m->L[l - 1].Ht;
-    g.ldb = m->B;
-    g.M = Ly.out;
-    g.N = Ly.in_pad;
-    g.K = m->B;
-    g.Cf = Ly.gW;
-    g.ldc = Ly.in_pad;
-    if (int ierr = gemm<EPI_STORE>(m, g)) return ierr;
-    hipLaunchKernelGGL(k_bias_grad, dim3((Ly.out + 255) / 256), dim3(256), 0, m->stream, Ly.dZt, m->B, Ly.out, Ly.gb);
-    if (l > 0) {
-      MlpLayer &Lp = m->L[l - 1];
-      GemmArgs h = {};
-      h.A = Ly.dZ;
-      h.lda = Ly.out;
-      h.B = Ly.Wtb;
-      h.ldb = Ly.out;
-      h.M = m->B;
-      h.N = Ly.in_pad;
-      h.K = Ly.out;
-      h.Zprev = Lp.Z;
-      h.ldc = Lp.out;
-      h.Cb = Lp.dZ;
-      h.Cbt = Lp.dZt;
-      h.ldt = m->B;
-      if (int ierr = gemm<EPI_DGELU>(m, h)) return ierr;
-    }
+    MlpLayer &Lp = m->L[l - 1];
+    GemmArgs h = {};
+    h.A = Ly.dZ;
+    h.lda = Ly.out;
+    h.B = Ly.Wtb;
+    h.ldb = Ly.out;
+    h.M = m->B;
+    h.N = Ly.in_pad;
+    h.K = Ly.out;
+    h.Zprev = Lp.Z;
+    h.ldc = Lp.out;
+    h.Cb = Lp.dZ;
+    h.Cbt = Lp.dZt;
+    h.ldt = m->B;
+    if (int ierr = gemm<EPI_DGELU>(m, h)) return ierr;
   }
   MCHK(hipGetLastError());
   return SE2W_OK;
 }
 
-int adam(se2w_mlp *m, float lr) {
+// The Adam step number t + 1 at learning rate lr.
+AdamArgs next_adam(se2w_mlp *m, float lr) {
   m->t++;
   AdamArgs a;
   a.lr = lr;
@@ -428,6 +542,28 @@ int adam(se2w_mlp *m, float lr) {
   a.wd = m->weight_decay;
   a.bc1 = (float)(1.0 - std::pow(0.9, (double)m->t));
   a.bc2 = (float)(1.0 - std::pow(0.999, (double)m->t));
+  return a;
+}
+
+// All parameter gradients of the batch into gW, gb.
+int weight_gradients(se2w_mlp *m) {
+  hipLaunchKernelGGL(k_wgrad<false>, dim3(m->wgrad_blocks), dim3(256), 0, m->stream, (const WgradLayer *)m->wgrad,
+                     m->nl, m->B, AdamArgs{});
+  MCHK(hipGetLastError());
+  return SE2W_OK;
+}
+
+// The same gradients, applied as one Adam step.
+int weight_update(se2w_mlp *m, float lr) {
+  hipLaunchKernelGGL(k_wgrad<true>, dim3(m->wgrad_blocks), dim3(256), 0, m->stream, (const WgradLayer *)m->wgrad,
+                     m->nl, m->B, next_adam(m, lr));
+  MCHK(hipGetLastError());
+  return SE2W_OK;
+}
+
+// One Adam step from the stored gradients gW, gb.
+int adam(se2w_mlp *m, float lr) {
+  const AdamArgs a = next_adam(m, lr);
   for (MlpLayer &Ly : m->L) {
     hipLaunchKernelGGL(k_adam_w, dim3(Ly.in_pad / 32, Ly.out / 32), dim3(256), 0, m->stream, Ly.W, Ly.mW, Ly.vW,
                        (const float *)Ly.gW, Ly.out, Ly.in_pad, a, Ly.Wb, Ly.Wtb);
@@ -536,6 +672,18 @@ int se2w_mlp_create(int32_t nlayers, const int32_t *widths, int32_t batch, uint6
                 (ierr = malloc_zero(m, &m->Ts, (size_t)batch * m->out)) || (ierr = malloc_zero(m, &m->idx, batch)) ||
                 (ierr = malloc_zero(m, &m->part, m->nparts)) || (ierr = malloc_zero(m, &m->acc, 1))))
     ;
+  if (!ierr && !(ierr = malloc_zero(m, &m->wgrad, nlayers))) {
+    std::vector<WgradLayer> wl(nlayers);
+    for (int l = 0; l < nlayers; l++) {
+      const MlpLayer &Ly = m->L[l];
+      wl[l] = WgradLayer{Ly.dZt, l == 0 ? m->H0t : m->L[l - 1].Ht, Ly.out, Ly.in_pad, m->wgrad_blocks,
+                         Ly.W,   Ly.mW, Ly.vW, Ly.gW, Ly.b, Ly.mb, Ly.vb, Ly.gb, Ly.Wb, Ly.Wtb};
+      m->wgrad_blocks += (Ly.out / 64) * (Ly.in_pad / 64) + (Ly.out + 255) / 256;
+    }
+    if (hipMemcpyAsync(m->wgrad, wl.data(), sizeof(WgradLayer) * nlayers, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
+        hipStreamSynchronize(m->stream) != hipSuccess)
+      ierr = mfail(SE2W_ERR_HIP, "layer table upload failed");
+  }
   if (!ierr) ierr = refresh_bf16(m);
   if (ierr) {
     se2w_mlp_destroy(m);
@@ -625,6 +773,7 @@ int se2w_mlp_gradient(se2w_mlp *m, int32_t n, const float *x, const float *targe
   MCHK(hipMemsetAsync(m->acc, 0, sizeof(double), m->stream));
   if (int ierr = forward(m)) return ierr;
   if (int ierr = backward(m, 0, 1.0 / ((double)m->B * m->out))) return ierr;
+  if (int ierr = weight_gradients(m)) return ierr;
   double l = 0.0;
   MCHK(hipMemcpyAsync(&l, m->acc, sizeof(double), hipMemcpyDeviceToHost, m->stream));
   std::vector<float *> w, b;
@@ -706,7 +855,7 @@ int se2w_mlp_train(se2w_mlp *m, int32_t epochs, float lr, uint64_t shuffle_seed,
         // cosine decay: lr_s = lr (1 + cos(pi s / S)) / 2 over the S steps of this call
         const double frac = (double)(e * nb + k) / ((double)epochs * nb);
         const float lr_s = m->cosine ? (float)(0.5 * lr * (1.0 + std::cos(3.14159265358979323846 * frac))) : lr;
-        ierr = adam(m, lr_s);
+        ierr = weight_update(m, lr_s);
       }
     }
   }

@@ -50,18 +50,25 @@ __device__ __forceinline__ float gelu_grad(float z) {
   return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
-enum { EPI_GELU = 0, EPI_LINEAR = 1, EPI_DGELU = 2 };
+enum { EPI_GELU = 0, EPI_LINEAR = 1, EPI_DGELU = 2, EPI_LOSS = 3 };
 
 struct GemmArgs {
   const bf16 *A;  // [M][lda]
   const bf16 *B;  // [N][ldb]
   int M, N, K, lda, ldb;
-  const float *bias;   // [N]          (EPI_GELU, EPI_LINEAR)
-  float *Cf;           // [M][ldc]     FP32 result (pre-activation or gradient)
+  const float *bias;   // [N]          (all but EPI_DGELU)
+  float *Cf;           // [M][ldc]     FP32 result: pre-activation (EPI_GELU), output (EPI_LINEAR)
   bf16 *Cb;            // [M][ldc]     BF16 activation / gradient
   bf16 *Cbt;           // [N][ldt]     its transpose
   const float *Zprev;  // [M][ldc]     pre-activation whose GELU' scales the product (EPI_DGELU)
   int ldc, ldt;
+  // EPI_LOSS: the mean-squared error against rows idx[m] of T and its
+  // gradient scale (C + bias - T) as Cb, Cbt; each workgroup's sum of squares
+  // to part[its linear index]
+  const float *T;
+  const int *idx;
+  float scale;
+  double *part;
 };
 
 // A workgroup of WM x WN waves, each forming TM x TN MFMA tiles of 16 x 16
@@ -133,16 +140,24 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_nt(GemmArgs g) {
 #pragma unroll
       for (int r = 0; r < 4; r++) ct[wm + 16 * i + 4 * (lane >> 4) + r][wn + 16 * j + (lane & 15)] = acc[i][j][r];
   __syncthreads();
+  [[maybe_unused]] double sq = 0.0;
   for (int q = tid; q < MT * NT / 4; q += THREADS) {
     const int lm = q / (NT / 4), ln = 4 * (q % (NT / 4));
     floatx4 c = *(const floatx4 *)&ct[lm][ln];
     const int n = n0 + ln;
     const long o = (long)(m0 + lm) * g.ldc + n;
-    if constexpr (EPI == EPI_GELU || EPI == EPI_LINEAR) c += *(const floatx4 *)(g.bias + n);
-    if constexpr (EPI != EPI_DGELU) *(floatx4 *)(g.Cf + o) = c;
-    if constexpr (EPI == EPI_GELU || EPI == EPI_DGELU) {
+    if constexpr (EPI != EPI_DGELU) c += *(const floatx4 *)(g.bias + n);
+    if constexpr (EPI == EPI_GELU || EPI == EPI_LINEAR) *(floatx4 *)(g.Cf + o) = c;
+    if constexpr (EPI != EPI_LINEAR) {
       bf16x4 h;
-      if constexpr (EPI == EPI_DGELU) {
+      if constexpr (EPI == EPI_LOSS) {
+        const floatx4 d = c - *(const floatx4 *)(g.T + (long)g.idx[m0 + lm] * g.ldc + n);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          sq += (double)d[r] * d[r];
+          h[r] = (bf16)(g.scale * d[r]);
+        }
+      } else if constexpr (EPI == EPI_DGELU) {
         const floatx4 z = *(const floatx4 *)(g.Zprev + o);
 #pragma unroll
         for (int r = 0; r < 4; r++) h[r] = (bf16)(c[r] * gelu_grad(z[r]));
@@ -155,19 +170,29 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_nt(GemmArgs g) {
       for (int r = 0; r < 4; r++) tr[ln + r][lm] = h[r];
     }
   }
-  if constexpr (EPI == EPI_GELU || EPI == EPI_DGELU) {
+  if constexpr (EPI != EPI_LINEAR) {
     __syncthreads();
     for (int q = tid; q < MT * NT / 8; q += THREADS) {
       const int ln = q / (MT / 8), lm = 8 * (q % (MT / 8));
       *(bf16x8 *)(g.Cbt + (long)(n0 + ln) * g.ldt + m0 + lm) = *(const bf16x8 *)&tr[ln][lm];
     }
   }
+  if constexpr (EPI == EPI_LOSS) {
+    __shared__ double red[WM * WN];
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1) sq += __shfl_down(sq, w);
+    if (lane == 0) red[wave] = sq;
+    __syncthreads();
+    if (tid == 0) {
+      for (int w = 1; w < WM * WN; w++) sq += red[w];
+      g.part[blockIdx.y * gridDim.x + blockIdx.x] = sq;
+    }
+  }
 }
 
 // Batch gather: rows idx[r] of the FP32 data become the BF16 input
-// activations (and their transpose) and the FP32 targets of the batch.
-__global__ void k_gather(const float *X, const float *T, const int *idx, int B, int in_pad, int out, bf16 *H0,
-                         bf16 *H0t, float *Tb) {
+// activations and their transpose (the targets are read in place by the loss).
+__global__ void k_gather(const float *X, const int *idx, int B, int in_pad, bf16 *H0, bf16 *H0t) {
   const int r = blockIdx.x;
   const long src = idx[r];
   for (int k = threadIdx.x; k < in_pad; k += blockDim.x) {
@@ -175,41 +200,20 @@ __global__ void k_gather(const float *X, const float *T, const int *idx, int B, 
     H0[(long)r * in_pad + k] = h;
     H0t[(long)k * B + r] = h;
   }
-  if (T)
-    for (int k = threadIdx.x; k < out; k += blockDim.x) Tb[(long)r * out + k] = T[src * out + k];
 }
 
-// Mean-squared error: dY = 2 (Y - T) / (B N) as BF16 (and transpose); the
-// per-block sums of (Y - T)^2 go to part[] (summed in order afterwards).
-__global__ __launch_bounds__(256) void k_loss(const float *Y, const float *Tb, int B, int N, float scale, bf16 *dZ,
-                                              bf16 *dZt, double *part) {
+// *out = inv_count times the sum of part[0..n), one workgroup, fixed order.
+__global__ __launch_bounds__(256) void k_sum_parts(const double *part, long n, double inv_count, double *out) {
   __shared__ double red[256];
   double s = 0.0;
-  const long n = (long)B * N;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-    const int m = (int)(i / N), c = (int)(i - (long)m * N);
-    const float d = Y[i] - Tb[i];
-    s += (double)d * d;
-    const bf16 g = (bf16)(scale * d);
-    dZ[i] = g;
-    dZt[(long)c * B + m] = g;
-  }
+  for (long i = threadIdx.x; i < n; i += 256) s += part[i];
   red[threadIdx.x] = s;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-// acc[slot] += sum of part[0..n) (one thread, fixed order), divided by count.
-__global__ void k_sum_parts(const double *part, int n, double inv_count, double *acc, int slot) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    double s = 0.0;
-    for (int i = 0; i < n; i++) s += part[i];
-    acc[slot] += s * inv_count;
-  }
+  if (threadIdx.x == 0) *out = red[0] * inv_count;
 }
 
 struct AdamArgs {
@@ -420,15 +424,21 @@ struct se2w_mlp {
   int device = 0, nl = 0, B = 0, in = 0, in_pad = 0, out = 0;
   std::vector<MlpLayer> L;
   bf16 *H0 = nullptr, *H0t = nullptr;
-  float *Y = nullptr, *Tb = nullptr;
+  float *Y = nullptr;
   float *Xs = nullptr, *Ts = nullptr;  // staging of one host batch
   int *idx = nullptr;                  // batch row indices
   WgradLayer *wgrad = nullptr;         // [nl] the grouped weight kernel's layers
   int wgrad_blocks = 0;
   float *X = nullptr, *T = nullptr;    // training data
   int ndata = 0;
-  double *part = nullptr, *acc = nullptr;
-  int nparts = 0;
+  // per-workgroup squared errors of the batches of an epoch, nparts each
+  double *part = nullptr;
+  int nparts = 0, part_batches = 0;
+  double *loss = nullptr;  // loss of one batch (se2w_mlp_gradient)
+  // two permutations (this epoch's and the next one's), device and pinned
+  int *perm_dev = nullptr, *perm_host = nullptr;
+  size_t perm_cap = 0;  // entries of one
+  hipEvent_t perm_up[2] = {nullptr, nullptr};
   hipStream_t stream = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   long t = 0;  // Adam steps taken
@@ -456,22 +466,35 @@ int malloc_zero(se2w_mlp *m, T **p, size_t n) {
 // 32 x 32 when that does, else 16 x 16 with one wave per workgroup: a smaller
 // tile re-reads the operands more often, a larger one leaves CUs idle.
 constexpr int kCUs = 256;
+int tile_of(int M, int N) {
+  const long tiles64 = (long)(M / 64) * (N / 64);
+  return tiles64 >= kCUs ? 64 : 4 * tiles64 >= kCUs ? 32 : 16;
+}
 template <int EPI>
 int gemm(se2w_mlp *m, const GemmArgs &g) {
   if (g.M % 64 || g.N % 64 || g.K % 32 || g.lda % 8 || g.ldb % 8)
     return mfail(SE2W_ERR_ARG, "product shape %d x %d x %d not tileable", g.M, g.N, g.K);
-  const long tiles64 = (long)(g.M / 64) * (g.N / 64);
-  if (tiles64 >= kCUs)
+  const int tile = tile_of(g.M, g.N);
+  if (tile == 64)
     hipLaunchKernelGGL((gemm_nt<EPI, 2, 2, 2, 2>), dim3(g.N / 64, g.M / 64), dim3(256), 0, m->stream, g);
-  else if (4 * tiles64 >= kCUs)
+  else if (tile == 32)
     hipLaunchKernelGGL((gemm_nt<EPI, 1, 1, 2, 2>), dim3(g.N / 32, g.M / 32), dim3(256), 0, m->stream, g);
   else
     hipLaunchKernelGGL((gemm_nt<EPI, 1, 1, 1, 1>), dim3(g.N / 16, g.M / 16), dim3(64), 0, m->stream, g);
   return SE2W_OK;
 }
 
-// Forward pass of the batch in H0/H0t; output pre-activations in Y.
-int forward(se2w_mlp *m) {
+// Targets and outputs of a batch's loss.
+struct LossArgs {
+  const float *T;   // [rows][out]
+  const int *idx;   // [B] the batch's rows
+  double *part;     // [nparts]
+};
+
+// Forward pass of the batch in H0/H0t.  The outputs go to Y or, with a loss,
+// their error's gradient to the last layer's dZ, dZt and the squared errors
+// to part; the outputs themselves are then not stored.
+int forward(se2w_mlp *m, const LossArgs *loss) {
   for (int l = 0; l < m->nl; l++) {
     MlpLayer &Ly = m->L[l];
     GemmArgs g = {};
@@ -491,6 +514,15 @@ int forward(se2w_mlp *m) {
       g.Cbt = Ly.Ht;
       g.ldt = m->B;
       ierr = gemm<EPI_GELU>(m, g);
+    } else if (loss) {
+      g.Cb = Ly.dZ;
+      g.Cbt = Ly.dZt;
+      g.ldt = m->B;
+      g.T = loss->T;
+      g.idx = loss->idx;
+      g.part = loss->part;
+      g.scale = 2.0f / ((float)m->B * (float)m->out);
+      ierr = gemm<EPI_LOSS>(m, g);
     } else {
       g.Cf = m->Y;
       ierr = gemm<EPI_LINEAR>(m, g);
@@ -501,14 +533,8 @@ int forward(se2w_mlp *m) {
   return SE2W_OK;
 }
 
-// Loss of the batch (added to acc[slot] / count) and the gradient of every
-// pre-activation.
-int backward(se2w_mlp *m, int slot, double inv_count) {
-  MlpLayer &Lo = m->L[m->nl - 1];
-  const float scale = 2.0f / ((float)m->B * (float)m->out);
-  hipLaunchKernelGGL(k_loss, dim3(m->nparts), dim3(256), 0, m->stream, m->Y, m->Tb, m->B, m->out, scale, Lo.dZ,
-                     Lo.dZt, m->part);
-  hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(64), 0, m->stream, m->part, m->nparts, inv_count, m->acc, slot);
+// The gradient of every hidden pre-activation from the last layer's.
+int backward(se2w_mlp *m) {
   for (int l = m->nl - 1; l > 0; l--) {
     MlpLayer &Ly = m->L[l];
     MlpLayer &Lp = m->L[l - 1];
@@ -584,9 +610,38 @@ int stage_batch(se2w_mlp *m, int n, const float *x, const float *t) {
   std::vector<int> id(m->B);
   for (int r = 0; r < m->B; r++) id[r] = r;
   MCHK(hipMemcpyAsync(m->idx, id.data(), sizeof(int) * m->B, hipMemcpyHostToDevice, m->stream));
-  hipLaunchKernelGGL(k_gather, dim3(m->B), dim3(128), 0, m->stream, m->Xs, t ? m->Ts : nullptr, m->idx, m->B,
-                     m->in_pad, m->out, m->H0, m->H0t, m->Tb);
+  hipLaunchKernelGGL(k_gather, dim3(m->B), dim3(128), 0, m->stream, (const float *)m->Xs, (const int *)m->idx, m->B,
+                     m->in_pad, m->H0, m->H0t);
   MCHK(hipStreamSynchronize(m->stream));  // the host vectors above go out of scope
+  return SE2W_OK;
+}
+
+// Squared-error sums of `batches` batches.
+int ensure_parts(se2w_mlp *m, int batches) {
+  if (batches <= m->part_batches) return SE2W_OK;
+  if (m->part) hipFree(m->part);
+  m->part = nullptr;
+  m->part_batches = 0;
+  if (hipMalloc(&m->part, sizeof(double) * (size_t)batches * m->nparts) != hipSuccess) {
+    m->part = nullptr;
+    return mfail(SE2W_ERR_MEM, "hipMalloc failed");
+  }
+  m->part_batches = batches;
+  return SE2W_OK;
+}
+
+// Both permutation buffers, n entries each.
+int ensure_perm(se2w_mlp *m, size_t n) {
+  for (hipEvent_t &e : m->perm_up)
+    if (!e) MCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  if (n <= m->perm_cap) return SE2W_OK;
+  if (m->perm_dev) hipFree(m->perm_dev);
+  if (m->perm_host) hipHostFree(m->perm_host);
+  m->perm_dev = m->perm_host = nullptr;
+  m->perm_cap = 0;
+  MCHK(hipMalloc(&m->perm_dev, 2 * sizeof(int) * n));
+  MCHK(hipHostMalloc((void **)&m->perm_host, 2 * sizeof(int) * n, hipHostMallocDefault));
+  m->perm_cap = n;
   return SE2W_OK;
 }
 
@@ -663,14 +718,13 @@ int se2w_mlp_create(int32_t nlayers, const int32_t *widths, int32_t batch, uint6
         hipStreamSynchronize(m->stream) != hipSuccess)
       ierr = mfail(SE2W_ERR_HIP, "weight upload failed");
   }
-  m->nparts = 256;
+  m->nparts = (batch / tile_of(batch, m->out)) * (m->out / tile_of(batch, m->out));
   if (!ierr && ((ierr = malloc_zero(m, &m->H0, (size_t)batch * m->in_pad)) ||
                 (ierr = malloc_zero(m, &m->H0t, (size_t)batch * m->in_pad)) ||
                 (ierr = malloc_zero(m, &m->Y, (size_t)batch * m->out)) ||
-                (ierr = malloc_zero(m, &m->Tb, (size_t)batch * m->out)) ||
                 (ierr = malloc_zero(m, &m->Xs, (size_t)batch * m->in_pad)) ||
                 (ierr = malloc_zero(m, &m->Ts, (size_t)batch * m->out)) || (ierr = malloc_zero(m, &m->idx, batch)) ||
-                (ierr = malloc_zero(m, &m->part, m->nparts)) || (ierr = malloc_zero(m, &m->acc, 1))))
+                (ierr = malloc_zero(m, &m->loss, 1)) || (ierr = ensure_parts(m, 1))))
     ;
   if (!ierr && !(ierr = malloc_zero(m, &m->wgrad, nlayers))) {
     std::vector<WgradLayer> wl(nlayers);
@@ -753,7 +807,7 @@ int se2w_mlp_forward(se2w_mlp *m, int32_t n, const float *x, float *y) {
     const int k = std::min(m->B, n - r0);
     if (int ierr = stage_batch(m, k, x + (size_t)r0 * m->in, nullptr)) return ierr;
     MCHK(hipEventRecord(m->e0, m->stream));
-    if (int ierr = forward(m)) return ierr;
+    if (int ierr = forward(m, nullptr)) return ierr;
     MCHK(hipEventRecord(m->e1, m->stream));
     MCHK(hipMemcpyAsync(y + (size_t)r0 * m->out, m->Y, sizeof(float) * (size_t)k * m->out, hipMemcpyDeviceToHost, m->stream));
     MCHK(hipStreamSynchronize(m->stream));
@@ -770,12 +824,14 @@ int se2w_mlp_gradient(se2w_mlp *m, int32_t n, const float *x, const float *targe
   if (n != m->B) return mfail(SE2W_ERR_ARG, "gradient batch must have %d rows", m->B);
   MCHK(hipSetDevice(m->device));
   if (int ierr = stage_batch(m, n, x, target)) return ierr;
-  MCHK(hipMemsetAsync(m->acc, 0, sizeof(double), m->stream));
-  if (int ierr = forward(m)) return ierr;
-  if (int ierr = backward(m, 0, 1.0 / ((double)m->B * m->out))) return ierr;
+  const LossArgs la{m->Ts, m->idx, m->part};
+  if (int ierr = forward(m, &la)) return ierr;
+  if (int ierr = backward(m)) return ierr;
+  hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, m->stream, (const double *)m->part, (long)m->nparts,
+                     1.0 / ((double)m->B * m->out), m->loss);
   if (int ierr = weight_gradients(m)) return ierr;
   double l = 0.0;
-  MCHK(hipMemcpyAsync(&l, m->acc, sizeof(double), hipMemcpyDeviceToHost, m->stream));
+  MCHK(hipMemcpyAsync(&l, m->loss, sizeof(double), hipMemcpyDeviceToHost, m->stream));
   std::vector<float *> w, b;
   for (MlpLayer &Ly : m->L) { w.push_back(Ly.gW); b.push_back(Ly.gb); }
   if (int ierr = params_copy(m, grad, true, w, b)) return ierr;
@@ -817,47 +873,50 @@ int se2w_mlp_train(se2w_mlp *m, int32_t epochs, float lr, uint64_t shuffle_seed,
   if (m->ndata < m->B) return mfail(SE2W_ERR_STATE, "set the training data first");
   MCHK(hipSetDevice(m->device));
   const int nb = m->ndata / m->B;
+  const size_t np = (size_t)nb * m->B;
+  if (int ierr = ensure_parts(m, nb)) return ierr;
+  if (int ierr = ensure_perm(m, np)) return ierr;
   std::vector<int> perm(m->ndata);
-  int *d_perm = nullptr;
   double *d_loss = nullptr;
-  MCHK(hipMalloc(&d_perm, sizeof(int) * (size_t)nb * m->B));
-  if (hipMalloc(&d_loss, sizeof(double) * epochs) != hipSuccess) {
-    hipFree(d_perm);
-    return mfail(SE2W_ERR_MEM, "hipMalloc failed");
-  }
+  if (hipMalloc(&d_loss, sizeof(double) * epochs) != hipSuccess) return mfail(SE2W_ERR_MEM, "hipMalloc failed");
   int ierr = SE2W_OK;
   uint64_t rng = shuffle_seed;
-  if (hipMemsetAsync(d_loss, 0, sizeof(double) * epochs, m->stream) != hipSuccess ||
-      hipEventRecord(m->e0, m->stream) != hipSuccess)
-    ierr = mfail(SE2W_ERR_HIP, "training setup failed");
+  if (hipEventRecord(m->e0, m->stream) != hipSuccess) ierr = mfail(SE2W_ERR_HIP, "training setup failed");
   for (int e = 0; e < epochs && !ierr; e++) {
     for (int i = 0; i < m->ndata; i++) perm[i] = i;
     for (int i = m->ndata - 1; i > 0; i--) {  // Fisher-Yates
       const int j = (int)(uniform01(rng) * (i + 1));
       std::swap(perm[i], perm[j]);
     }
-    // the previous epoch's kernels may still read d_perm
-    if (hipStreamSynchronize(m->stream) != hipSuccess ||
-        hipMemcpy(d_perm, perm.data(), sizeof(int) * (size_t)nb * m->B, hipMemcpyHostToDevice) != hipSuccess) {
+    // The permutation goes up on the stream, so the host may run an epoch
+    // ahead; the pinned half is free again once its previous copy has gone
+    // up (the device half is ordered by the stream).
+    const int half = e & 1;
+    int *hp = m->perm_host + half * m->perm_cap, *dp = m->perm_dev + half * m->perm_cap;
+    if (e >= 2 && hipEventSynchronize(m->perm_up[half]) != hipSuccess) {
+      ierr = mfail(SE2W_ERR_HIP, "permutation upload failed");
+      break;
+    }
+    memcpy(hp, perm.data(), sizeof(int) * np);
+    if (hipMemcpyAsync(dp, hp, sizeof(int) * np, hipMemcpyHostToDevice, m->stream) != hipSuccess ||
+        hipEventRecord(m->perm_up[half], m->stream) != hipSuccess) {
       ierr = mfail(SE2W_ERR_HIP, "permutation upload failed");
       break;
     }
     for (int k = 0; k < nb && !ierr; k++) {
-      hipLaunchKernelGGL(k_gather, dim3(m->B), dim3(128), 0, m->stream, (const float *)m->X, (const float *)m->T,
-                         (const int *)(d_perm + (size_t)k * m->B), m->B, m->in_pad, m->out, m->H0, m->H0t, m->Tb);
-      if ((ierr = forward(m))) break;
-      // each batch loss enters d_loss[e] as loss / nb
-      double *acc0 = m->acc;
-      m->acc = d_loss;
-      ierr = backward(m, e, 1.0 / ((double)m->B * m->out * nb));
-      m->acc = acc0;
-      if (!ierr) {
-        // cosine decay: lr_s = lr (1 + cos(pi s / S)) / 2 over the S steps of this call
-        const double frac = (double)(e * nb + k) / ((double)epochs * nb);
-        const float lr_s = m->cosine ? (float)(0.5 * lr * (1.0 + std::cos(3.14159265358979323846 * frac))) : lr;
-        ierr = weight_update(m, lr_s);
-      }
+      const int *rows = dp + (size_t)k * m->B;
+      hipLaunchKernelGGL(k_gather, dim3(m->B), dim3(128), 0, m->stream, (const float *)m->X, rows, m->B, m->in_pad,
+                         m->H0, m->H0t);
+      const LossArgs la{m->T, rows, m->part + (size_t)k * m->nparts};
+      if ((ierr = forward(m, &la)) || (ierr = backward(m))) break;
+      // cosine decay: lr_s = lr (1 + cos(pi s / S)) / 2 over the S steps of this call
+      const double frac = (double)(e * nb + k) / ((double)epochs * nb);
+      const float lr_s = m->cosine ? (float)(0.5 * lr * (1.0 + std::cos(3.14159265358979323846 * frac))) : lr;
+      ierr = weight_update(m, lr_s);
     }
+    // the epoch's loss is the mean of its batch losses
+    hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, m->stream, (const double *)m->part, (long)nb * m->nparts,
+                       1.0 / ((double)m->B * m->out * nb), d_loss + e);
   }
   if (!ierr) {
     if (hipEventRecord(m->e1, m->stream) != hipSuccess || hipStreamSynchronize(m->stream) != hipSuccess) {
@@ -874,7 +933,6 @@ int se2w_mlp_train(se2w_mlp *m, int32_t epochs, float lr, uint64_t shuffle_seed,
     }
   }
   hipStreamSynchronize(m->stream);
-  hipFree(d_perm);
   hipFree(d_loss);
   return ierr;
 }
@@ -905,6 +963,11 @@ int se2w_mlp_destroy(se2w_mlp *m) {
   for (void *p : m->allocs) hipFree(p);
   if (m->X) hipFree(m->X);
   if (m->T) hipFree(m->T);
+  if (m->part) hipFree(m->part);
+  if (m->perm_dev) hipFree(m->perm_dev);
+  if (m->perm_host) hipHostFree(m->perm_host);
+  for (hipEvent_t e : m->perm_up)
+    if (e) hipEventDestroy(e);
   if (m->e0) hipEventDestroy(m->e0);
   if (m->e1) hipEventDestroy(m->e1);
   if (m->stream) hipStreamDestroy(m->stream);

@@ -2,7 +2,7 @@
 // hand-written gfx950 kernels (include/se2w_mlp.h).
 //
 // Every product is one kernel shape, C[M][N] = sum_k A[M][k] B[N][k] with
-// both operands BF16 and K-contiguous, on v_mfma_f32_16x16x32_bf16 with FP32
+// both operands BF16 in MFMA order (op_index), on v_mfma_f32_16x16x32_bf16 with FP32
 // accumulation.  The three products of a layer (forward, input gradient,
 // weight gradient) all take that shape because the forward and backward
 // epilogues also write the transposes of the activations and of the
@@ -50,18 +50,28 @@ __device__ __forceinline__ float gelu_grad(float z) {
   return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
 }
 
+// BF16 operands are stored in MFMA order: the 16 x 32 block (r / 16, k / 32)
+// of an operand with K columns is 1 KB, lane l's eight values at 16 l bytes
+// (row l % 16, columns 8 (l / 16) .. +7 of the block).  An operand load of a
+// wave is then one contiguous KB.  From row-major storage neighbouring lanes
+// read 16 bytes of different rows, and the loads ran at 16 bytes per clock
+// and CU: a 256 x 1024 x 4096 product took 32.4 us instead of 12.1.
+__host__ __device__ constexpr long op_index(int r, int k, int K) {
+  return ((long)(r / 16) * (K / 32) + k / 32) * 512 + (16 * (k % 32 / 8) + r % 16) * 8 + k % 8;
+}
+
 enum { EPI_GELU = 0, EPI_LINEAR = 1, EPI_DGELU = 2, EPI_LOSS = 3 };
 
 struct GemmArgs {
-  const bf16 *A;  // [M][lda]
-  const bf16 *B;  // [N][ldb]
-  int M, N, K, lda, ldb;
+  const bf16 *A;  // M x K operand
+  const bf16 *B;  // N x K operand
+  int M, N, K;
   const float *bias;   // [N]          (all but EPI_DGELU)
-  float *Cf;           // [M][ldc]     FP32 result: pre-activation (EPI_GELU), output (EPI_LINEAR)
-  bf16 *Cb;            // [M][ldc]     BF16 activation / gradient
-  bf16 *Cbt;           // [N][ldt]     its transpose
-  const float *Zprev;  // [M][ldc]     pre-activation whose GELU' scales the product (EPI_DGELU)
-  int ldc, ldt;
+  float *Cf;           // [M][N]       FP32 result: pre-activation (EPI_GELU), output (EPI_LINEAR)
+  bf16 *Cb;            // M x N operand: BF16 activation / gradient
+  bf16 *Cbt;           // N x ldt operand: its transpose, ldt the batch
+  const float *Zprev;  // [M][N]       pre-activation whose GELU' scales the product (EPI_DGELU)
+  int ldt;
   // EPI_LOSS: the mean-squared error against rows idx[m] of T and its
   // gradient scale (C + bias - T) as Cb, Cbt; each workgroup's sum of squares
   // to part[its linear index]
@@ -79,8 +89,7 @@ struct GemmArgs {
 // steps already in flight; no barrier and no LDS round trip per step.  Every
 // element is one chain of products in ascending k, so its bits do not depend
 // on the tile shape.  The result goes through LDS once, so that the epilogue
-// reads and writes whole lines (16 bytes per lane along the rows, and along
-// the columns for the transpose).
+// reads and writes 16 bytes per lane.
 // MFMA 16x16x32 operand layout: lane l holds A[l % 16][8 (l / 16) .. +7] and
 // B[8 (l / 16) .. +7][l % 16] (B is stored [n][k], so also row l % 16, eight
 // consecutive k); the result D[4 (l / 16) + r][l % 16] is its r-th
@@ -89,7 +98,7 @@ template <int EPI, int TM, int TN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_nt(GemmArgs g) {
   constexpr int MT = 16 * TM * WM, NT = 16 * TN * WN, THREADS = 64 * WM * WN, U = 16 / (TM + TN);
   __shared__ __attribute__((aligned(16))) float ct[MT][NT + 4];
-  __shared__ __attribute__((aligned(16))) bf16 tr[NT][MT + 8];  // transposed BF16 result
+  __shared__ __attribute__((aligned(16))) bf16 th[MT][NT + 8], tr[NT][MT + 8];  // BF16 result and its transpose
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int m0 = blockIdx.y * MT, n0 = blockIdx.x * NT;
   const int wm = 16 * TM * (wave / WN), wn = 16 * TN * (wave % WN);
@@ -98,20 +107,20 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_nt(GemmArgs g) {
   for (int i = 0; i < TM; i++)
 #pragma unroll
     for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const bf16 *ga = g.A + (long)(m0 + wm + (lane & 15)) * g.lda + 8 * (lane >> 4);
-  const bf16 *gb = g.B + (long)(n0 + wn + (lane & 15)) * g.ldb + 8 * (lane >> 4);
   const int ks = g.K / 32;
+  const bf16 *ga = g.A + op_index(m0 + wm, 0, g.K) + 8 * lane;
+  const bf16 *gb = g.B + op_index(n0 + wn, 0, g.K) + 8 * lane;
   bf16x8 a[2][U][TM], b[2][U][TN];
   // loads of the steps k .. k + U - 1 (past the end the last step is read
   // again, and not multiplied)
   auto load = [&](int slot, int k) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const long o = 32l * min(k + u, ks - 1);
+      const int o = min(k + u, ks - 1);
 #pragma unroll
-      for (int i = 0; i < TM; i++) a[slot][u][i] = *(const bf16x8 *)(ga + (long)i * 16 * g.lda + o);
+      for (int i = 0; i < TM; i++) a[slot][u][i] = *(const bf16x8 *)(ga + 512l * (i * ks + o));
 #pragma unroll
-      for (int j = 0; j < TN; j++) b[slot][u][j] = *(const bf16x8 *)(gb + (long)j * 16 * g.ldb + o);
+      for (int j = 0; j < TN; j++) b[slot][u][j] = *(const bf16x8 *)(gb + 512l * (j * ks + o));
     }
   };
   auto multiply = [&](int slot, int k) {
@@ -145,13 +154,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_nt(GemmArgs g) {
     const int lm = q / (NT / 4), ln = 4 * (q % (NT / 4));
     floatx4 c = *(const floatx4 *)&ct[lm][ln];
     const int n = n0 + ln;
-    const long o = (long)(m0 + lm) * g.ldc + n;
+    const long o = (long)(m0 + lm) * g.N + n;
     if constexpr (EPI != EPI_DGELU) c += *(const floatx4 *)(g.bias + n);
     if constexpr (EPI == EPI_GELU || EPI == EPI_LINEAR) *(floatx4 *)(g.Cf + o) = c;
     if constexpr (EPI != EPI_LINEAR) {
       bf16x4 h;
       if constexpr (EPI == EPI_LOSS) {
-        const floatx4 d = c - *(const floatx4 *)(g.T + (long)g.idx[m0 + lm] * g.ldc + n);
+        const floatx4 d = c - *(const floatx4 *)(g.T + (long)g.idx[m0 + lm] * g.N + n);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
           sq += (double)d[r] * d[r];
@@ -165,16 +174,18 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_nt(GemmArgs g) {
 #pragma unroll
         for (int r = 0; r < 4; r++) h[r] = (bf16)gelu(c[r]);
       }
-      *(bf16x4 *)(g.Cb + o) = h;
+      *(bf16x4 *)&th[lm][ln] = h;
 #pragma unroll
       for (int r = 0; r < 4; r++) tr[ln + r][lm] = h[r];
     }
   }
   if constexpr (EPI != EPI_LINEAR) {
     __syncthreads();
-    for (int q = tid; q < MT * NT / 8; q += THREADS) {
-      const int ln = q / (MT / 8), lm = 8 * (q % (MT / 8));
-      *(bf16x8 *)(g.Cbt + (long)(n0 + ln) * g.ldt + m0 + lm) = *(const bf16x8 *)&tr[ln][lm];
+    for (int q = tid; q < MT * NT / 8; q += THREADS) {  // 16 rows of one 16-byte column piece at a time
+      const int c = 8 * (q / 16 % (NT / 8)), r = 16 * (q / (2 * NT)) + q % 16;
+      *(bf16x8 *)(g.Cb + op_index(m0 + r, n0 + c, g.N)) = *(const bf16x8 *)&th[r][c];
+      const int ct8 = 8 * (q / 16 % (MT / 8)), rt = 16 * (q / (2 * MT)) + q % 16;
+      *(bf16x8 *)(g.Cbt + op_index(n0 + rt, m0 + ct8, g.ldt)) = *(const bf16x8 *)&tr[rt][ct8];
     }
   }
   if constexpr (EPI == EPI_LOSS) {
@@ -197,8 +208,8 @@ __global__ void k_gather(const float *X, const int *idx, int B, int in_pad, bf16
   const long src = idx[r];
   for (int k = threadIdx.x; k < in_pad; k += blockDim.x) {
     const bf16 h = (bf16)X[src * in_pad + k];
-    H0[(long)r * in_pad + k] = h;
-    H0t[(long)k * B + r] = h;
+    H0[op_index(r, k, in_pad)] = h;
+    H0t[op_index(k, r, B)] = h;
   }
 }
 
@@ -231,7 +242,7 @@ __device__ __forceinline__ float adam_update(float &w, float &m, float &v, float
 }
 
 // Adam on a [rows][cols] weight matrix (rows, cols multiples of 32): FP32
-// master weights, BF16 copy W[rows][cols] and transposed copy Wt[cols][rows].
+// master weights, BF16 operand Wb (rows x cols) and its transpose Wtb.
 // A 32 x 32 tile per workgroup of 32 x 8 threads; the transpose goes through LDS.
 __global__ __launch_bounds__(256) void k_adam_w(float *W, float *m, float *v, const float *g, int rows, int cols,
                                                 AdamArgs a, bf16 *Wb, bf16 *Wtb) {
@@ -246,11 +257,11 @@ __global__ __launch_bounds__(256) void k_adam_w(float *W, float *m, float *v, co
     m[o] = mm;
     v[o] = vv;
     const bf16 h = (bf16)w;
-    Wb[o] = h;
+    Wb[op_index(r0 + k, c0 + tx, cols)] = h;
     tile[k][tx] = h;
   }
   __syncthreads();
-  for (int k = ty; k < 32; k += 8) Wtb[(long)(c0 + k) * rows + r0 + tx] = tile[tx][k];
+  for (int k = ty; k < 32; k += 8) Wtb[op_index(c0 + k, r0 + tx, rows)] = tile[tx][k];
 }
 
 __global__ void k_adam_b(float *b, float *m, float *v, const float *g, int n, AdamArgs a) {
@@ -265,8 +276,8 @@ __global__ void k_adam_b(float *b, float *m, float *v, const float *g, int n, Ad
 
 // One layer of the grouped weight kernel.
 struct WgradLayer {
-  const bf16 *dZt;  // [out][B]     gradient of the pre-activation, transposed
-  const bf16 *Ht;   // [in_pad][B]  the layer's input, transposed
+  const bf16 *dZt;  // out x B operand: gradient of the pre-activation, transposed
+  const bf16 *Ht;   // in_pad x B operand: the layer's input, transposed
   int out, in_pad;
   int tile0;        // its first workgroup; it has (out / 64) (in_pad / 64) tiles, then ceil(out / 256) bias blocks
   float *W, *mW, *vW, *gW, *b, *mb, *vb, *gb;
@@ -285,7 +296,7 @@ struct WgradLayer {
 template <bool ADAM>
 __global__ __launch_bounds__(256) void k_wgrad(const WgradLayer *layers, int nl, int B, AdamArgs a) {
   __shared__ __attribute__((aligned(16))) float gt[64][68];
-  __shared__ __attribute__((aligned(16))) bf16 tr[64][72];
+  __shared__ __attribute__((aligned(16))) bf16 th[64][72], tr[64][72];
   const int tid = threadIdx.x;
   int l = nl - 1;
   while (l > 0 && (int)blockIdx.x < layers[l].tile0) l--;
@@ -294,12 +305,12 @@ __global__ __launch_bounds__(256) void k_wgrad(const WgradLayer *layers, int nl,
   if (t >= nt) {  // bias block
     const int o = (t - nt) * 256 + tid;
     if (o >= L.out) return;
-    const bf16 *row = L.dZt + (long)o * B;
+    const bf16 *row = L.dZt + op_index(o, 0, B);  // eight values every 128, 512 per 32 columns
     float s = 0.f;
     for (int k = 0; k < B; k += 64) {
       bf16x8 x[8];
 #pragma unroll
-      for (int q = 0; q < 8; q++) x[q] = *(const bf16x8 *)(row + k + 8 * q);
+      for (int q = 0; q < 8; q++) x[q] = *(const bf16x8 *)(row + 16l * k + 128 * q);
 #pragma unroll
       for (int q = 0; q < 8; q++)
 #pragma unroll
@@ -335,16 +346,16 @@ __global__ __launch_bounds__(256) void k_wgrad(const WgradLayer *layers, int nl,
   for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  const bf16 *ga = L.dZt + (long)(m0 + wm + (lane & 15)) * B + 8 * (lane >> 4);
-  const bf16 *gb = L.Ht + (long)(n0 + wn + (lane & 15)) * B + 8 * (lane >> 4);
+  const bf16 *ga = L.dZt + op_index(m0 + wm, 0, B) + 8 * lane;
+  const bf16 *gb = L.Ht + op_index(n0 + wn, 0, B) + 8 * lane;
   for (int k = 0; k < B; k += 64) {  // B is a multiple of 64
     bf16x8 x[2][2], y[2][2];
 #pragma unroll
     for (int u = 0; u < 2; u++)
 #pragma unroll
       for (int i = 0; i < 2; i++) {
-        x[u][i] = *(const bf16x8 *)(ga + (long)i * 16 * B + k + 32 * u);
-        y[u][i] = *(const bf16x8 *)(gb + (long)i * 16 * B + k + 32 * u);
+        x[u][i] = *(const bf16x8 *)(ga + 16l * (i * B + k + 32 * u));
+        y[u][i] = *(const bf16x8 *)(gb + 16l * (i * B + k + 32 * u));
       }
 #pragma unroll
     for (int u = 0; u < 2; u++)
@@ -378,10 +389,10 @@ __global__ __launch_bounds__(256) void k_wgrad(const WgradLayer *layers, int nl,
         h[r] = (bf16)w;
         tr[ec + r][lm] = h[r];
       }
+      *(bf16x4 *)&th[lm][ec] = h;
       *(floatx4 *)(L.W + o) = w4[q];
       *(floatx4 *)(L.mW + o) = m4[q];
       *(floatx4 *)(L.vW + o) = v4[q];
-      *(bf16x4 *)(L.Wb + o) = h;
     } else {
       *(floatx4 *)(L.gW + o) = g;
     }
@@ -389,8 +400,9 @@ __global__ __launch_bounds__(256) void k_wgrad(const WgradLayer *layers, int nl,
   if constexpr (ADAM) {
     __syncthreads();
     for (int q = tid; q < 64 * 8; q += 256) {
-      const int ln = q >> 3, lm = 8 * (q & 7);
-      *(bf16x8 *)(L.Wtb + (long)(n0 + ln) * L.out + m0 + lm) = *(const bf16x8 *)&tr[ln][lm];
+      const int c = 8 * (q / 16 % 8), r = 16 * (q / 128) + q % 16;
+      *(bf16x8 *)(L.Wb + op_index(m0 + r, n0 + c, L.in_pad)) = *(const bf16x8 *)&th[r][c];
+      *(bf16x8 *)(L.Wtb + op_index(n0 + r, m0 + c, L.out)) = *(const bf16x8 *)&tr[r][c];
     }
   }
 }
@@ -401,8 +413,8 @@ __global__ void k_to_bf16(const float *W, int rows, int cols, bf16 *Wb, bf16 *Wt
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
     const int r = (int)(i / cols), c = (int)(i - (long)r * cols);
     const bf16 h = (bf16)W[i];
-    Wb[i] = h;
-    Wtb[(long)c * rows + r] = h;
+    Wb[op_index(r, c, cols)] = h;
+    Wtb[op_index(c, r, rows)] = h;
   }
 }
 
@@ -414,10 +426,10 @@ struct MlpLayer {
   int in = 0, in_pad = 0, out = 0;
   float *W = nullptr, *b = nullptr, *gW = nullptr, *gb = nullptr, *mW = nullptr, *vW = nullptr, *mb = nullptr,
         *vb = nullptr;
-  bf16 *Wb = nullptr, *Wtb = nullptr;
+  bf16 *Wb = nullptr, *Wtb = nullptr;        // out x in_pad operand and its transpose
   float *Z = nullptr;                        // pre-activation [B][out] (hidden layers)
-  bf16 *H = nullptr, *Ht = nullptr;          // activation [B][out], [out][B] (hidden layers)
-  bf16 *dZ = nullptr, *dZt = nullptr;        // d loss / d pre-activation [B][out], [out][B]
+  bf16 *H = nullptr, *Ht = nullptr;          // activation, B x out operand and its transpose (hidden layers)
+  bf16 *dZ = nullptr, *dZt = nullptr;        // d loss / d pre-activation, likewise
 };
 
 struct se2w_mlp {
@@ -472,7 +484,7 @@ int tile_of(int M, int N) {
 }
 template <int EPI>
 int gemm(se2w_mlp *m, const GemmArgs &g) {
-  if (g.M % 64 || g.N % 64 || g.K % 32 || g.lda % 8 || g.ldb % 8)
+  if (g.M % 64 || g.N % 64 || g.K % 64)
     return mfail(SE2W_ERR_ARG, "product shape %d x %d x %d not tileable", g.M, g.N, g.K);
   const int tile = tile_of(g.M, g.N);
   if (tile == 64)
@@ -499,25 +511,21 @@ int forward(se2w_mlp *m, const LossArgs *loss) {
     MlpLayer &Ly = m->L[l];
     GemmArgs g = {};
     g.A = l == 0 ? m->H0 : m->L[l - 1].H;
-    g.lda = Ly.in_pad;
     g.B = Ly.Wb;
-    g.ldb = Ly.in_pad;
     g.M = m->B;
     g.N = Ly.out;
     g.K = Ly.in_pad;
     g.bias = Ly.b;
-    g.ldc = Ly.out;
+    g.ldt = m->B;
     int ierr;
     if (l < m->nl - 1) {
       g.Cf = Ly.Z;
       g.Cb = Ly.H;
       g.Cbt = Ly.Ht;
-      g.ldt = m->B;
       ierr = gemm<EPI_GELU>(m, g);
     } else if (loss) {
       g.Cb = Ly.dZ;
       g.Cbt = Ly.dZt;
-      g.ldt = m->B;
       g.T = loss->T;
       g.idx = loss->idx;
       g.part = loss->part;
@@ -540,14 +548,11 @@ int backward(se2w_mlp *m) {
     MlpLayer &Lp = m->L[l - 1];
     GemmArgs h = {};
     h.A = Ly.dZ;
-    h.lda = Ly.out;
     h.B = Ly.Wtb;
-    h.ldb = Ly.out;
     h.M = m->B;
     h.N = Ly.in_pad;
     h.K = Ly.out;
     h.Zprev = Lp.Z;
-    h.ldc = Lp.out;
     h.Cb = Lp.dZ;
     h.Cbt = Lp.dZt;
     h.ldt = m->B;

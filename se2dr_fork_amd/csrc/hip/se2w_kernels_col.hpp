@@ -1,0 +1,300 @@
+// se2w_kernels_col.hpp -- column kernel: one lane per element column.
+//
+// The p + 1 lanes of an element each hold one column of its nodes and the
+// quadrature points of that column (lane i: the points (i, qj) and the nodes
+// (i, j)).  A wave holds 64 / (p + 1) neighbouring elements of one element
+// row, a workgroup WX waves in x times EY element rows.  Sums along a column
+// (d/dy of the displacement, the column terms of the forces) run in the lane's
+// registers against a derivative table that is the same for the whole wave,
+// in SGPRs; sums along a row read the element's other columns from LDS, where
+// every lane of an element reads the same address.  An element's rows are
+// exchanged three times inside its wave (displacement, row stresses, nodal
+// forces, all in one buffer, without a barrier); one barrier lets the
+// neighbours' edge forces through.
+//
+// What it is for: from p = 5 up a lane or lane pair per element (the register
+// kernels) holds 2 (p+1)^2 values per component, which takes a SIMD's whole
+// register file in FP64 (one wave, scratch traffic from p = 7 on), and small
+// meshes give such a kernel too few waves.  Here a lane holds a few times
+// p + 1 values, and a mesh gives (p+1)/2 times the waves.
+//
+// Every sum runs over the same terms in the same order, with the same
+// roundings, as in reg64_body / reg_body, so the results have the same bits
+// (FP64: those of the reference's loop).  One exception: the diagonal terms
+// of a row sum (the node or point of the lane's own column) are added through
+// a multiply-add with a factor 1 or 0, which differs from adding them on that
+// one lane only when the term is infinite, that is after an overflow of the
+// displacement.
+//
+// Tiling: as in the register kernels, a workgroup owns its elements except
+// the left column and the bottom row, which only supply their edge forces;
+// the waves of the bottom row form the top edge alone.  The owner lane of a
+// node updates it: lanes run along the node rows, so the loads and stores are
+// contiguous except for the column that neighbouring elements share.
+#pragma once
+#include "se2w_kernels.hpp"
+
+namespace se2w {
+
+// Schedules: waves in x, element rows, minimum waves per SIMD.
+struct ColSchedule { int wx, ey, waves; };
+constexpr ColSchedule kColSchedules[] = {{1, 4, 3}, {1, 8, 3}};
+constexpr int kNumColSchedules = sizeof(kColSchedules) / sizeof(kColSchedules[0]);
+constexpr int col_epw(int p) { return 64 / (p + 1); }  // elements per wave
+constexpr bool col_schedule_built(int P, int S, bool fused) {
+  return fused && P >= 2 && P <= kMaxP && S >= 0 && S < kNumColSchedules;
+}
+
+// Orders the LDS accesses of one wave: its LDS instructions execute in order,
+// so only the compiler has to keep them in order.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int P, int MODE, int WX, int EY, typename PRM>
+__device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last) {
+#pragma clang fp contract(off)
+  using R = typename RealOf<MODE>::T;
+  using R2 = typename V2<R>::T;
+  using CR = const __attribute__((address_space(4))) R;
+  constexpr int NB = P + 1, EPW = col_epw(P), EX = EPW * WX;
+  constexpr int TEX = EX - 1, TEY = EY - 1;
+  // An odd number of nodes per element: the elements of a wave read rows at
+  // this stride, which then falls on different banks.
+  constexpr int ES = (NB * NB) | 1;
+  __shared__ R2 buf[EY][EX][ES];
+
+  const int tx = tile % prm.tiles_x, ty = tile / prm.tiles_x;
+  const int ex0 = tx * TEX, ey0 = ty * TEY;
+  const int ex_end = min(ex0 + TEX, prm.mx), ey_end = min(ey0 + TEY, prm.my);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  // Lanes past the wave's last whole element repeat the last lane and store
+  // nothing to memory.
+  const int el = min(lane / NB, EPW - 1), i = min(lane - el * NB, P);
+  const int ly = wave / WX, lx = (wave % WX) * EPW + el;
+  const int ey = ey0 - 1 + ly, ex = ex0 - 1 + lx;
+  const bool row_valid = ey >= 0 && ey < ey_end;  // uniform per wave
+  const bool owner = row_valid && ly >= 1 && lx >= 1 && ex < ex_end && lane < EPW * NB;
+  R2 *B = &buf[ly][lx][0];  // [j][i]
+
+  R2 F[NB];  // forces of the nodes (i, j)
+  if (row_valid) {
+    // columns of elements outside the mesh repeat its first or last column of
+    // elements; nobody uses their forces
+    const int exc = min(max(ex, 0), prm.mx - 1);
+    const long base = (long)(ey * P) * prm.pitch + exc * P + i;
+    R2 u[NB];
+#pragma unroll
+    for (int j = 0; j < NB; j++) u[j] = prm.u_in[base + (long)j * prm.pitch];
+    const int e = exc + ey * prm.mx;
+    const R J00 = R(0.5) * prm.elem_dx[exc], J11 = R(0.5) * prm.elem_dy[ey];
+    const R iJ00 = R(1) / J00, iJ11 = R(1) / J11, detJ = J00 * J11;
+    const R lam = prm.lambda[e], mu = prm.mu[e], c11 = R(2) * mu + lam;
+    CR *D = (CR *)(uintptr_t)prm.D;
+    CR *W = (CR *)(uintptr_t)prm.w2;
+#pragma unroll
+    for (int j = 0; j < NB; j++) B[j * NB + i] = u[j];
+    // derivatives along a row: at the lane's points dr[k] (of node column k),
+    // at the lane's nodes dc[k] (from point column k)
+    R dr[NB], dc[NB], w[NB];
+#pragma unroll
+    for (int k = 0; k < NB; k++) {
+      dr[k] = prm.D[i * NB + k];
+      dc[k] = prm.D[k * NB + i];
+      w[k] = prm.w2[i + k * NB];
+    }
+    wave_lds_order();
+    if constexpr (MODE == MODE_F64) {
+      // dN_dy of the element row, iJ11 D[qj][j], formed once on the host
+      CR *dny = (CR *)(uintptr_t)prm.dny + (long)ey * (NB * NB);
+      R own[NB];  // 1 for the lane's own column
+#pragma unroll
+      for (int k = 0; k < NB; k++) {
+        dr[k] = iJ00 * dr[k];
+        dc[k] = iJ00 * dc[k];
+        own[k] = k == i ? R(1) : R(0);
+      }
+      R sxx[NB], sxy[NB], syy[NB];
+#pragma unroll
+      for (int qj = 0; qj < NB; qj++) {
+        R e0 = R(0), e1 = R(0), e2 = R(0);
+#pragma unroll
+        for (int j = 0; j < qj; j++) {
+          e1 = e1 + dny[qj * NB + j] * u[j].y;
+          e2 = e2 + dny[qj * NB + j] * u[j].x;
+        }
+        e1 = e1 + dny[qj * NB + qj] * u[qj].y;
+        const R tq = dny[qj * NB + qj] * u[qj].x;
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+          const R2 uk = B[qj * NB + k];
+          e0 = e0 + dr[k] * uk.x;
+          e2 = e2 + fma(own[k], tq, dr[k] * uk.y);
+        }
+#pragma unroll
+        for (int j = qj + 1; j < NB; j++) {
+          e1 = e1 + dny[qj * NB + j] * u[j].y;
+          e2 = e2 + dny[qj * NB + j] * u[j].x;
+        }
+        sxx[qj] = c11 * e0 + lam * e1;
+        syy[qj] = lam * e0 + c11 * e1;
+        sxy[qj] = mu * e2;
+      }
+      wave_lds_order();
+#pragma unroll
+      for (int qj = 0; qj < NB; qj++) B[qj * NB + i] = R2{sxx[qj], sxy[qj]};
+      wave_lds_order();
+      // row terms of node row j: points (k, j), k ascending, the lane's own
+      // point with its column term inside
+      auto row_terms = [&](int j, R2 &f) {
+        const R cx = dny[j * NB + j] * sxy[j], cy = dny[j * NB + j] * syy[j];
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+          const R2 s = B[j * NB + k];
+          const R nfac = -(detJ * W[k + j * NB]);
+          f.x = f.x + nfac * fma(own[k], cx, dc[k] * s.x);
+          f.y = f.y + nfac * fma(own[k], cy, dc[k] * s.y);
+        }
+      };
+      auto column_term = [&](int qj, int j, R2 &f) {
+        const R nfac = -(detJ * w[qj]);
+        f.x = f.x + nfac * (dny[qj * NB + j] * sxy[qj]);
+        f.y = f.y + nfac * (dny[qj * NB + j] * syy[qj]);
+      };
+      if (ly == 0) {  // uniform per wave
+        R2 f = R2{R(0), R(0)};
+#pragma unroll
+        for (int qj = 0; qj < P; qj++) column_term(qj, P, f);
+        row_terms(P, f);
+        F[P] = f;
+      } else {
+#pragma unroll
+        for (int j = 0; j < NB; j++) F[j] = R2{R(0), R(0)};
+#pragma unroll
+        for (int qj = 0; qj < NB; qj++) {
+          row_terms(qj, F[qj]);
+#pragma unroll
+          for (int j = 0; j < NB; j++)
+            if (j != qj) column_term(qj, j, F[j]);
+        }
+      }
+    } else {
+      const R s = -detJ;
+      const R a1 = s * c11 * iJ00 * iJ00, a2 = s * lam * iJ00 * iJ11, a3 = s * c11 * iJ11 * iJ11;
+      const R b1 = s * mu * iJ11 * iJ11, b2 = s * mu * iJ00 * iJ11, b3 = s * mu * iJ00 * iJ00;
+      // row stresses (A, Cx) and column stresses (Bs, E), as in
+      // RegOperator::row_stress
+      R2 rs[NB], cs[NB];
+#pragma unroll
+      for (int qj = 0; qj < NB; qj++) {
+        R dxux = R(0), dxuy = R(0), dyux = R(0), dyuy = R(0);
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+          const R2 uk = B[qj * NB + k];
+          dxux = fma(dr[k], uk.x, dxux);
+          dxuy = fma(dr[k], uk.y, dxuy);
+          dyux = fma((R)D[qj * NB + k], u[k].x, dyux);
+          dyuy = fma((R)D[qj * NB + k], u[k].y, dyuy);
+        }
+        rs[qj] = R2{w[qj] * fma(a1, dxux, a2 * dyuy), w[qj] * fma(b3, dxuy, b2 * dyux)};
+        cs[qj] = R2{w[qj] * fma(b1, dyux, b2 * dxuy), w[qj] * fma(a3, dyuy, a2 * dxux)};
+      }
+      wave_lds_order();
+#pragma unroll
+      for (int qj = 0; qj < NB; qj++) B[qj * NB + i] = rs[qj];
+      wave_lds_order();
+      auto row_terms = [&](int j, R2 &f) {
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+          const R2 t = B[j * NB + k];
+          f.x = fma(dc[k], t.x, f.x);
+          f.y = fma(dc[k], t.y, f.y);
+        }
+      };
+      auto column_term = [&](int qj, int j, R2 &f) {
+        f.x = fma((R)D[qj * NB + j], cs[qj].x, f.x);
+        f.y = fma((R)D[qj * NB + j], cs[qj].y, f.y);
+      };
+      if (ly == 0) {
+        R2 f = R2{R(0), R(0)};
+#pragma unroll
+        for (int qj = 0; qj < P; qj++) column_term(qj, P, f);
+        row_terms(P, f);
+        column_term(P, P, f);
+        F[P] = f;
+      } else {
+#pragma unroll
+        for (int j = 0; j < NB; j++) F[j] = R2{R(0), R(0)};
+#pragma unroll
+        for (int qj = 0; qj < NB; qj++) {
+          row_terms(qj, F[qj]);
+#pragma unroll
+          for (int j = 0; j < NB; j++) column_term(qj, j, F[j]);
+        }
+      }
+    }
+    // The edges that the neighbours read: node column p (i = p) and node row
+    // p, where the rows' stresses were.
+    wave_lds_order();
+    if (ly != 0) {
+#pragma unroll
+      for (int j = 0; j < P; j++)
+        if (i == P) B[j * NB + P] = F[j];
+    }
+    B[P * NB + i] = F[P];
+  }
+  // The update's loads go out before the barrier; nodes that the lane does
+  // not own load an owned node instead (in bounds, unused), so they carry no
+  // branch.
+  const bool rb = ex == prm.mx - 1, tb = ey == prm.my - 1;  // domain right / top boundary
+  const bool mine = owner && (i < P || rb);
+  const int gx = mine ? ex * P + i : ex0 * P;
+  const int gy0 = mine ? ey * P : ey0 * P;
+  const long idx0 = (long)gy0 * prm.pitch + gx;
+  R2 pu[NB], pv[NB], pc[NB];
+  R pm[NB];
+#pragma unroll
+  for (int j = 0; j < NB; j++) {
+    const long idx = idx0 + (long)(j < P || (mine && tb) ? j : 0) * prm.pitch;
+    pu[j] = prm.u_in[idx];
+    pv[j] = prm.v[idx];
+    pm[j] = prm.mass[idx];
+    if constexpr (MODE == MODE_F32K) pc[j] = prm.c_in[idx];
+    else pc[j] = R2{R(0), R(0)};
+  }
+  const TileLists tl = tile_lists(prm, tile, step, last);
+  __syncthreads();
+  if (!mine) return;
+  const bool left = ex > 0 && i == 0, below = ey > 0;
+  // the own force and the neighbours' in ascending element order
+  const R2 *L = &buf[ly][lx - 1][0], *Dn = &buf[ly - 1][lx][0], *Dg = &buf[ly - 1][lx - 1][0];
+#pragma unroll
+  for (int j = 0; j < NB; j++) {
+    if (j == P && !tb) break;
+    R2 g = F[j];
+    if (j == 0 && below) {
+      R2 t = Dn[P * NB + i];
+      if (left) {  // (ex-1,ey-1), (ex,ey-1), (ex-1,ey), own
+        const R2 d = Dg[P * NB + P], l = L[P];
+        t = R2{(d.x + t.x) + l.x, (d.y + t.y) + l.y};
+      }
+      g = R2{t.x + g.x, t.y + g.y};
+    } else if (left) {
+      const R2 l = L[j * NB + P];
+      g = R2{l.x + g.x, l.y + g.y};
+    }
+    node_update_core<P, MODE>(prm, tl, gx, gy0 + j, idx0 + (long)j * prm.pitch, g.x, g.y, pu[j].x, pu[j].y, pv[j],
+                              pm[j], pc[j]);
+  }
+}
+
+template <int P, int MODE, int WX, int EY, int WAVES>
+__global__ __launch_bounds__(64 * WX * EY) __attribute__((amdgpu_waves_per_eu(WAVES, 8)))
+void col_kernel(StepParams<typename RealOf<MODE>::T> prm) {
+  const int tile = tile_of_block(blockIdx.x, prm.tiles_per_xcd);
+  if (tile >= prm.tiles_x * prm.tiles_y) return;  // uniform per workgroup
+  col_body<P, MODE, WX, EY>(prm, tile, prm.step, prm.last);
+}
+
+}  // namespace se2w

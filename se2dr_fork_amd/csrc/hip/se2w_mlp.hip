@@ -213,6 +213,22 @@ __global__ void k_gather(const float *X, const int *idx, int B, int in_pad, bf16
   }
 }
 
+// Rows of a forward batch, read in place from pinned host memory (a batch is
+// some tens of KB; its upload by a copy command took longer than the network
+// for one row): rows x[n][in] become the input operand, zero in the padding
+// and in the rows past n.
+__global__ void k_rows(const float *x, int n, int in, int in_pad, bf16 *H0) {
+  const int r = blockIdx.x;
+  for (int k = threadIdx.x; k < in_pad; k += blockDim.x)
+    H0[op_index(r, k, in_pad)] = (bf16)(r < n && k < in ? x[(long)r * in + k] : 0.f);
+}
+
+// Download of n 16-byte pieces into pinned host memory: queued behind the
+// product like any kernel, where a copy command waits for another engine.
+__global__ __launch_bounds__(256) void k_to_host(const floatx4 *src, floatx4 *dst, long n) {
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) dst[i] = src[i];
+}
+
 // *out = inv_count times the sum of part[0..n), one workgroup, fixed order.
 __global__ __launch_bounds__(256) void k_sum_parts(const double *part, long n, double inv_count, double *out) {
   __shared__ double red[256];
@@ -432,6 +448,9 @@ struct MlpLayer {
   bf16 *dZ = nullptr, *dZt = nullptr;        // d loss / d pre-activation, likewise
 };
 
+// Output chunks that se2w_mlp_forward keeps in flight.
+constexpr int kAhead = 4;
+
 struct se2w_mlp {
   int device = 0, nl = 0, B = 0, in = 0, in_pad = 0, out = 0;
   std::vector<MlpLayer> L;
@@ -446,6 +465,10 @@ struct se2w_mlp {
   // per-workgroup squared errors of the batches of an epoch, nparts each
   double *part = nullptr;
   int nparts = 0, part_batches = 0;
+  // se2w_mlp_forward's pinned buffers: the input rows of kAhead + 1 batches
+  // and kAhead chunks of chunk_rows() output rows, with the events of each
+  float *x_host = nullptr, *y_host = nullptr;
+  hipEvent_t y_up[kAhead] = {}, f0[kAhead + 1] = {}, f1[kAhead + 1] = {};
   double *loss = nullptr;  // loss of one batch (se2w_mlp_gradient)
   // two permutations (this epoch's and the next one's), device and pinned
   int *perm_dev = nullptr, *perm_host = nullptr;
@@ -479,12 +502,12 @@ int malloc_zero(se2w_mlp *m, T **p, size_t n) {
 // tile re-reads the operands more often, a larger one leaves CUs idle.
 constexpr int kCUs = 256;
 int tile_of(int M, int N) {
-  const long tiles64 = (long)(M / 64) * (N / 64);
-  return tiles64 >= kCUs ? 64 : 4 * tiles64 >= kCUs ? 32 : 16;
+  const long tiles16 = (long)(M / 16) * (N / 16);
+  return M % 64 == 0 && tiles16 >= 16 * kCUs ? 64 : M % 32 == 0 && tiles16 >= 4 * kCUs ? 32 : 16;
 }
 template <int EPI>
 int gemm(se2w_mlp *m, const GemmArgs &g) {
-  if (g.M % 64 || g.N % 64 || g.K % 64)
+  if (g.M % 16 || g.N % 64 || g.K % 64)
     return mfail(SE2W_ERR_ARG, "product shape %d x %d x %d not tileable", g.M, g.N, g.K);
   const int tile = tile_of(g.M, g.N);
   if (tile == 64)
@@ -503,16 +526,16 @@ struct LossArgs {
   double *part;     // [nparts]
 };
 
-// Forward pass of the batch in H0/H0t.  The outputs go to Y or, with a loss,
-// their error's gradient to the last layer's dZ, dZt and the squared errors
-// to part; the outputs themselves are then not stored.
-int forward(se2w_mlp *m, const LossArgs *loss) {
+// Forward pass of the first `rows` rows in H0.  The outputs go to Y or, with a
+// loss (rows = the batch), their error's gradient to the last layer's dZ, dZt
+// and the squared errors to part; the outputs themselves are then not stored.
+int forward(se2w_mlp *m, int rows, const LossArgs *loss, float *Y) {
   for (int l = 0; l < m->nl; l++) {
     MlpLayer &Ly = m->L[l];
     GemmArgs g = {};
     g.A = l == 0 ? m->H0 : m->L[l - 1].H;
     g.B = Ly.Wb;
-    g.M = m->B;
+    g.M = rows;
     g.N = Ly.out;
     g.K = Ly.in_pad;
     g.bias = Ly.b;
@@ -532,7 +555,7 @@ int forward(se2w_mlp *m, const LossArgs *loss) {
       g.scale = 2.0f / ((float)m->B * (float)m->out);
       ierr = gemm<EPI_LOSS>(m, g);
     } else {
-      g.Cf = m->Y;
+      g.Cf = Y;
       ierr = gemm<EPI_LINEAR>(m, g);
     }
     if (ierr) return ierr;
@@ -632,6 +655,32 @@ int ensure_parts(se2w_mlp *m, int batches) {
     return mfail(SE2W_ERR_MEM, "hipMalloc failed");
   }
   m->part_batches = batches;
+  return SE2W_OK;
+}
+
+// Output rows of one downloaded chunk: about 1 MB, so that the copy out of a
+// chunk hides behind the next chunks' downloads, and at least the 16 rows that
+// a product writes at once.
+int chunk_rows(const se2w_mlp *m) { return std::min(m->B, std::max(16, (1 << 18) / m->out)); }
+
+int forward_buffers(se2w_mlp *m) {
+  for (hipEvent_t &e : m->y_up)
+    if (!e) MCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  for (int s = 0; s <= kAhead; s++) {
+    if (!m->f0[s]) MCHK(hipEventCreate(&m->f0[s]));
+    if (!m->f1[s]) MCHK(hipEventCreate(&m->f1[s]));
+  }
+  // Filled once: the host's first touch of a pinned page costs a fault each,
+  // which the first forward would pay.
+  const size_t nx = (size_t)(kAhead + 1) * m->B * m->in, ny = (size_t)kAhead * chunk_rows(m) * m->out;
+  if (!m->x_host) {
+    MCHK(hipHostMalloc((void **)&m->x_host, sizeof(float) * nx, hipHostMallocDefault));
+    memset(m->x_host, 0, sizeof(float) * nx);
+  }
+  if (!m->y_host) {
+    MCHK(hipHostMalloc((void **)&m->y_host, sizeof(float) * ny, hipHostMallocDefault));
+    memset(m->y_host, 0, sizeof(float) * ny);
+  }
   return SE2W_OK;
 }
 
@@ -743,6 +792,7 @@ int se2w_mlp_create(int32_t nlayers, const int32_t *widths, int32_t batch, uint6
         hipStreamSynchronize(m->stream) != hipSuccess)
       ierr = mfail(SE2W_ERR_HIP, "layer table upload failed");
   }
+  if (!ierr) ierr = forward_buffers(m);
   if (!ierr) ierr = refresh_bf16(m);
   if (ierr) {
     se2w_mlp_destroy(m);
@@ -760,19 +810,34 @@ int se2w_mlp_param_count(se2w_mlp *m, int64_t *count) {
   return SE2W_OK;
 }
 
-// copy between the packed host layout and the padded device weights
-static int params_copy(se2w_mlp *m, float *host, bool to_host, const std::vector<float *> &src_w,
-                       const std::vector<float *> &src_b) {
+// Copy between the packed host layout and the padded device weights.  Rows
+// are padded only where the input width is not a multiple of 64 (the first
+// layer): that matrix goes through a padded host copy in one piece, since a
+// 2D copy of pageable memory moves row by row (48 ms for 1024 rows).
+static int params_copy(se2w_mlp *m, float *host, bool to_host, const std::vector<float *> &dev_w,
+                       const std::vector<float *> &dev_b) {
+  std::vector<float> padded;
+  const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
+  auto copy = [&](float *h, float *d, size_t n) {
+    return hipMemcpyAsync(to_host ? h : d, to_host ? d : h, sizeof(float) * n, kind, m->stream);
+  };
   size_t off = 0;
   for (int l = 0; l < m->nl; l++) {
     const MlpLayer &Ly = m->L[l];
-    MCHK(hipMemcpy2DAsync(to_host ? (void *)(host + off) : (void *)src_w[l], to_host ? sizeof(float) * Ly.in : sizeof(float) * Ly.in_pad,
-                          to_host ? (const void *)src_w[l] : (const void *)(host + off),
-                          to_host ? sizeof(float) * Ly.in_pad : sizeof(float) * Ly.in, sizeof(float) * Ly.in, Ly.out,
-                          to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, m->stream));
+    float *w = host + off;
+    if (Ly.in == Ly.in_pad) {
+      MCHK(copy(w, dev_w[l], (size_t)Ly.out * Ly.in));
+    } else {
+      padded.assign((size_t)Ly.out * Ly.in_pad, 0.f);
+      if (!to_host)
+        for (int o = 0; o < Ly.out; o++) memcpy(&padded[(size_t)o * Ly.in_pad], w + (size_t)o * Ly.in, sizeof(float) * Ly.in);
+      MCHK(copy(padded.data(), dev_w[l], padded.size()));
+      MCHK(hipStreamSynchronize(m->stream));
+      if (to_host)
+        for (int o = 0; o < Ly.out; o++) memcpy(w + (size_t)o * Ly.in, &padded[(size_t)o * Ly.in_pad], sizeof(float) * Ly.in);
+    }
     off += (size_t)Ly.out * Ly.in;
-    MCHK(hipMemcpyAsync(to_host ? (void *)(host + off) : (void *)src_b[l], to_host ? (const void *)src_b[l] : (const void *)(host + off),
-                        sizeof(float) * Ly.out, to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, m->stream));
+    MCHK(copy(host + off, dev_b[l], Ly.out));
     off += Ly.out;
   }
   MCHK(hipStreamSynchronize(m->stream));
@@ -807,20 +872,53 @@ int se2w_mlp_set_params(se2w_mlp *m, const float *params) {
 int se2w_mlp_forward(se2w_mlp *m, int32_t n, const float *x, float *y) {
   if (!m || n < 0 || (n > 0 && (!x || !y))) return mfail(SE2W_ERR_ARG, "bad forward arguments");
   MCHK(hipSetDevice(m->device));
-  float total = 0.f;
-  for (int r0 = 0; r0 < n; r0 += m->B) {
-    const int k = std::min(m->B, n - r0);
-    if (int ierr = stage_batch(m, k, x + (size_t)r0 * m->in, nullptr)) return ierr;
-    MCHK(hipEventRecord(m->e0, m->stream));
-    if (int ierr = forward(m, nullptr)) return ierr;
-    MCHK(hipEventRecord(m->e1, m->stream));
-    MCHK(hipMemcpyAsync(y + (size_t)r0 * m->out, m->Y, sizeof(float) * (size_t)k * m->out, hipMemcpyDeviceToHost, m->stream));
-    MCHK(hipStreamSynchronize(m->stream));
-    float ms = 0.f;
-    MCHK(hipEventElapsedTime(&ms, m->e0, m->e1));
-    total += ms;
+  m->fwd_ms = 0.0;
+  if (n == 0) return SE2W_OK;
+  // a call that ended on an error may have left work that uses the buffers
+  MCHK(hipStreamSynchronize(m->stream));
+  // Batches in order on the stream, each followed by the download of its
+  // chunks; chunk c is handed over once chunk c - kAhead has been copied out,
+  // so a batch's products and the next chunks' downloads run while the host
+  // copies the earlier ones out.
+  const int cr = chunk_rows(m), per = (m->B + cr - 1) / cr;  // chunks of a whole batch
+  const int nchunks = n / m->B * per + (n % m->B + cr - 1) / cr;
+  auto enqueue = [&](int c) -> int {
+    const int b = c / per, s = b % (kAhead + 1), r0 = b * m->B, k = std::min(m->B, n - r0);
+    const int c0 = (c % per) * cr, rows = std::min(cr, k - c0);
+    float *slot = m->y_host + (size_t)(c % kAhead) * cr * m->out;
+    // few rows are written to the pinned chunk by the last product itself
+    const bool direct = k <= 16;
+    if (c % per == 0) {
+      float *xh = m->x_host + (size_t)s * m->B * m->in;
+      memcpy(xh, x + (size_t)r0 * m->in, sizeof(float) * (size_t)k * m->in);
+      const int M = k <= 16 ? 16 : k <= 32 ? 32 : round_up(k, 64);
+      MCHK(hipEventRecord(m->f0[s], m->stream));
+      hipLaunchKernelGGL(k_rows, dim3(M), dim3(128), 0, m->stream, (const float *)xh, k, m->in, m->in_pad, m->H0);
+      if (int ierr = forward(m, M, nullptr, direct ? slot : m->Y)) return ierr;
+      MCHK(hipEventRecord(m->f1[s], m->stream));
+    }
+    if (!direct)
+      hipLaunchKernelGGL(k_to_host, dim3(128), dim3(256), 0, m->stream, (const floatx4 *)(m->Y + (size_t)c0 * m->out),
+                         (floatx4 *)slot, (long)rows * m->out / 4);
+    MCHK(hipEventRecord(m->y_up[c % kAhead], m->stream));
+    return SE2W_OK;
+  };
+  for (int c = 0; c < std::min(kAhead, nchunks); c++)
+    if (int ierr = enqueue(c)) return ierr;
+  for (int c = 0; c < nchunks; c++) {
+    const int b = c / per, s = b % (kAhead + 1), r0 = b * m->B, k = std::min(m->B, n - r0);
+    const int c0 = (c % per) * cr, rows = std::min(cr, k - c0);
+    MCHK(hipEventSynchronize(m->y_up[c % kAhead]));
+    memcpy(y + (size_t)(r0 + c0) * m->out, m->y_host + (size_t)(c % kAhead) * cr * m->out,
+           sizeof(float) * (size_t)rows * m->out);
+    if (c % per == 0) {
+      float ms = 0.f;
+      MCHK(hipEventElapsedTime(&ms, m->f0[s], m->f1[s]));
+      m->fwd_ms += ms;
+    }
+    if (c + kAhead < nchunks)
+      if (int ierr = enqueue(c + kAhead)) return ierr;
   }
-  m->fwd_ms = total;
   return SE2W_OK;
 }
 
@@ -830,7 +928,7 @@ int se2w_mlp_gradient(se2w_mlp *m, int32_t n, const float *x, const float *targe
   MCHK(hipSetDevice(m->device));
   if (int ierr = stage_batch(m, n, x, target)) return ierr;
   const LossArgs la{m->Ts, m->idx, m->part};
-  if (int ierr = forward(m, &la)) return ierr;
+  if (int ierr = forward(m, m->B, &la, nullptr)) return ierr;
   if (int ierr = backward(m)) return ierr;
   hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(256), 0, m->stream, (const double *)m->part, (long)m->nparts,
                      1.0 / ((double)m->B * m->out), m->loss);
@@ -864,9 +962,9 @@ int se2w_mlp_set_data(se2w_mlp *m, int32_t n, const float *x, const float *targe
   m->ndata = 0;
   MCHK(hipMalloc(&m->X, sizeof(float) * (size_t)n * m->in_pad));
   MCHK(hipMalloc(&m->T, sizeof(float) * (size_t)n * m->out));
-  MCHK(hipMemset2DAsync(m->X, sizeof(float) * m->in_pad, 0, sizeof(float) * m->in_pad, n, m->stream));
-  MCHK(hipMemcpy2DAsync(m->X, sizeof(float) * m->in_pad, x, sizeof(float) * m->in, sizeof(float) * m->in, n,
-                        hipMemcpyHostToDevice, m->stream));
+  std::vector<float> padded((size_t)n * m->in_pad, 0.f);  // in one piece, as in params_copy
+  for (int r = 0; r < n; r++) memcpy(&padded[(size_t)r * m->in_pad], x + (size_t)r * m->in, sizeof(float) * m->in);
+  MCHK(hipMemcpyAsync(m->X, padded.data(), sizeof(float) * padded.size(), hipMemcpyHostToDevice, m->stream));
   MCHK(hipMemcpyAsync(m->T, target, sizeof(float) * (size_t)n * m->out, hipMemcpyHostToDevice, m->stream));
   MCHK(hipStreamSynchronize(m->stream));
   m->ndata = n;
@@ -913,7 +1011,7 @@ int se2w_mlp_train(se2w_mlp *m, int32_t epochs, float lr, uint64_t shuffle_seed,
       hipLaunchKernelGGL(k_gather, dim3(m->B), dim3(128), 0, m->stream, (const float *)m->X, rows, m->B, m->in_pad,
                          m->H0, m->H0t);
       const LossArgs la{m->T, rows, m->part + (size_t)k * m->nparts};
-      if ((ierr = forward(m, &la)) || (ierr = backward(m))) break;
+      if ((ierr = forward(m, m->B, &la, nullptr)) || (ierr = backward(m))) break;
       // cosine decay: lr_s = lr (1 + cos(pi s / S)) / 2 over the S steps of this call
       const double frac = (double)(e * nb + k) / ((double)epochs * nb);
       const float lr_s = m->cosine ? (float)(0.5 * lr * (1.0 + std::cos(3.14159265358979323846 * frac))) : lr;
@@ -968,6 +1066,14 @@ int se2w_mlp_destroy(se2w_mlp *m) {
   for (void *p : m->allocs) hipFree(p);
   if (m->X) hipFree(m->X);
   if (m->T) hipFree(m->T);
+  if (m->x_host) hipHostFree(m->x_host);
+  if (m->y_host) hipHostFree(m->y_host);
+  for (hipEvent_t e : m->y_up)
+    if (e) hipEventDestroy(e);
+  for (int s = 0; s <= kAhead; s++) {
+    if (m->f0[s]) hipEventDestroy(m->f0[s]);
+    if (m->f1[s]) hipEventDestroy(m->f1[s]);
+  }
   if (m->part) hipFree(m->part);
   if (m->perm_dev) hipFree(m->perm_dev);
   if (m->perm_host) hipHostFree(m->perm_host);

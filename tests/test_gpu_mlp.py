@@ -103,3 +103,43 @@ def test_mlp_argument_errors():
     with pytest.raises(S.Se2wError, match="training data"):
         m.train(1)
     m.close()
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64, 65, 129, 300])
+def test_forward_rows_at_the_edges_of_tiles_and_chunks(rows):
+    """Row counts on both sides of the row tiles (16, 32, 64), of a batch and
+    of the downloaded chunks; a row's result does not depend on the others."""
+    m = S.Mlp(SMALL, batch=128, seed=5)
+    x = np.random.default_rng(3).standard_normal((rows, SMALL[0])).astype(np.float32)
+    y = m.forward(x)
+    y0, _ = M.forward(m.params(), SMALL, x)
+    assert rel_l2(y, y0) < 5e-3
+    np.testing.assert_array_equal(m.forward(x[-1:]), y[-1:])
+    m.close()
+
+
+@pytest.mark.parametrize("widths,batch", [([66, 64, 64], 64), (SMALL, 192), ([1, 320, 64, 128], 128)])
+def test_a_training_step_is_its_gradient_and_one_adam_step(widths, batch):
+    """One batch trained equals the stored gradient of the same (shuffled)
+    rows followed by one Adam step, bit for bit: the grouped kernel forms and
+    applies the gradients in the order in which the gradient entry stores
+    them."""
+    rng = np.random.default_rng(6)
+    x = rng.standard_normal((batch, widths[0])).astype(np.float32)
+    t = rng.standard_normal((batch, widths[-1])).astype(np.float32)
+    s, mask, order = 7, (1 << 64) - 1, list(range(batch))
+    for i in range(batch - 1, 0, -1):  # Fisher-Yates on a splitmix64 stream
+        s = (s + 0x9E3779B97F4A7C15) & mask
+        z = ((s ^ (s >> 30)) * 0xBF58476D1CE4E5B9) & mask
+        z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & mask
+        j = int(((z ^ (z >> 31)) >> 11) * (1.0 / 9007199254740992.0) * (i + 1))
+        order[i], order[j] = order[j], order[i]
+    a, b = S.Mlp(widths, batch=batch, seed=8), S.Mlp(widths, batch=batch, seed=8)
+    a.set_data(x, t)
+    loss = a.train(1, lr=1e-3, seed=7)[0]
+    loss_b, g = b.gradient(x[order], t[order])
+    b.adam_step(g, 1e-3)
+    np.testing.assert_array_equal(a.params(), b.params())
+    assert loss == pytest.approx(loss_b, rel=1e-6)
+    a.close()
+    b.close()

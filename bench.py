@@ -118,6 +118,10 @@ REG_SCHEDULES = [(32, 4, 0, 4, 1), (64, 2, 0, 4, 1), (32, 2, 0, 2, 1), (32, 4, 0
 REG64_SCHEDULES = [(32, 4, 3, 0, 2), (32, 4, 0, 0, 2), (16, 8, 0, 4, 2), (32, 4, 3, 4, 2), (32, 4, 2, 0, 1),
                    (64, 2, 2, 0, 1), (32, 4, 2, 4, 1), (16, 4, 1, 4, 2), (32, 4, 1, 4, 2)]
 KERNEL_REG64 = 12
+# (waves in x, element rows) of the column kernel's schedules
+# (SE2W_KERNEL_COL + k)
+COL_SCHEDULES = [(1, 4), (1, 8)]
+KERNEL_COL = 21
 
 
 def kernel_signature(variant, p, mode):
@@ -130,6 +134,9 @@ def kernel_signature(variant, p, mode):
         return f"line_kernel<{p}, {mode}>"
     if variant == 11:
         return f"tile_kernel<{p}, {mode}, true, 512>"
+    if variant >= KERNEL_COL:
+        wx, ey = COL_SCHEDULES[variant - KERNEL_COL]
+        return f"col_kernel<{p}, {mode}, {wx}, {ey}>"
     if variant >= KERNEL_REG64:
         ex, ey, w, pf, lpe = REG64_SCHEDULES[variant - KERNEL_REG64]
         return f"reg64_kernel<{p}, {ex}, {ey}, {w}, {pf}, {lpe}>"
@@ -147,6 +154,9 @@ def ens_kernel_signature(variant, p, mode):
         return f"ens_line_kernel<{p}, {mode}>"
     if variant == 11:
         return f"ens_tile_kernel<{p}, {mode}, 512>"
+    if variant >= KERNEL_COL:
+        wx, ey = COL_SCHEDULES[variant - KERNEL_COL]
+        return f"ens_col_kernel<{p}, {mode}, {wx}, {ey}>"
     if variant >= KERNEL_REG64:
         ex, ey, w, pf, lpe = REG64_SCHEDULES[variant - KERNEL_REG64]
         return f"ens_reg64_kernel<{p}, {ex}, {ey}, {w}, {pf}, {lpe}>"
@@ -157,6 +167,8 @@ def ens_kernel_signature(variant, p, mode):
 def kernel_name(variant, p, mode):
     what = ("LDS-staged tile" if variant == 0 else "matrix-core contractions" if variant == 9 else
             "line contractions" if variant == 10 else "LDS-staged tile, 512 threads" if variant == 11 else
+            "lane per element column, %d element rows" % COL_SCHEDULES[variant - KERNEL_COL][1]
+            if variant >= KERNEL_COL else
             "FP64 %s per element in the reference's operation order, %dx%d elements" %
             (("lane", "lane pair")[REG64_SCHEDULES[variant - KERNEL_REG64][4] - 1],
              *REG64_SCHEDULES[variant - KERNEL_REG64][:2]) if variant >= KERNEL_REG64 else

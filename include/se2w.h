@@ -183,6 +183,8 @@ int se2w_get_timing(se2w_ctx *ctx, double *run_ms, double kernel_ms[2]);
                                 order, first schedule; SE2W_KERNEL_REG64 + k for the k-th (nine in all: a lane
                                 pair or one lane per element, several tile shapes; above p = 4 the lane pairs;
                                 k = 0..6 up to p = 7, k = 7, 8 at p = 8, one wave per SIMD) */
+#define SE2W_KERNEL_COL 21 /* all modes, 2 <= p <= 8, fused: column kernel, one lane per element column;
+                              SE2W_KERNEL_COL + k for the k-th workgroup shape (two in all, FP64 the first) */
 
 /* Selects / reports the element-kernel variant (no counterpart in the
  * reference: a schedule choice of this implementation, used by the
@@ -192,8 +194,8 @@ int se2w_get_kernel(se2w_ctx *ctx, int32_t *variant);
 int se2w_kernel_count(void);
 
 /* Autotuner (no counterpart in the reference): runs `reps` timed trials of
- * `steps` steps for every element-kernel variant built for this context's
- * degree, precision and schedule, keeps the fastest (median kernel time) and
+ * `steps` steps for every element-kernel variant that is the fastest on some
+ * mesh at this context's degree, precision and schedule, keeps the fastest (median kernel time) and
  * reports it.  The state u, v, a is restored afterwards; receiver rows of the
  * previous se2w_run are discarded.  The choice is cached per (p, precision,
  * schedule, size bucket) for the rest of the process. */

@@ -16,6 +16,7 @@
 
 #include "se2w.h"
 #include "se2w_kernels.hpp"
+#include "se2w_kernels_col.hpp"
 #include "se2w_kernels_reg.hpp"
 #include "se2w_kernels_mfma.hpp"
 #include "se2w_kernels_reg64.hpp"
@@ -176,7 +177,7 @@ struct se2w_ctx {
   bool pred_ok = false;
   double pred_dt = 0.0;
   void *mass = nullptr, *lambda = nullptr, *mu = nullptr, *edx = nullptr, *edy = nullptr, *D = nullptr,
-       *w2 = nullptr;
+       *w2 = nullptr, *dny = nullptr;
   int cur = 0;
   bool have_tables = false, have_cells = false, have_mass = false;
   // host copies needed for receiver post-processing
@@ -287,6 +288,30 @@ bool reg64_variant_built(int p, int mode, int variant, int schedule) {
          reg64_schedule_built(p, variant - SE2W_KERNEL_REG64, schedule == SE2W_SCHED_FUSED);
 }
 
+// variant = SE2W_KERNEL_COL + schedule index into kColSchedules (all modes)
+static_assert(SE2W_KERNEL_COL == SE2W_KERNEL_REG64 + kNumReg64Schedules, "variant numbering");
+constexpr int kNumVariants = SE2W_KERNEL_COL + kNumColSchedules;
+bool is_col_variant(int variant) { return variant >= SE2W_KERNEL_COL && variant < kNumVariants; }
+bool col_variant_built(int p, int mode, int variant, int schedule) {
+  return is_col_variant(variant) && col_schedule_built(p, mode, variant - SE2W_KERNEL_COL, schedule == SE2W_SCHED_FUSED);
+}
+
+// Variants that an autotuner times: those that are the fastest on some mesh.
+// The LDS kernels are behind from p = 2 on, the matrix-core and line kernels
+// everywhere, and in FP64 the register kernels from p = 5 on (the column
+// kernel is 1.4 to 3 times as fast from 24 x 24 elements to 389 x 389).  Below,
+// in FP64, the column kernel leads up to a million nodes (256 x 256 p4: 22.6
+// against 26.1 us) and trails on large meshes (800 x 800 p4: 211 against 189
+// us), where a short trial can mistake it for the faster one: two million is
+// the line.  The kernels that are left have the same bits, so a tuned run does
+// not depend on the choice.
+bool tuning_candidate(int p, int mode, int schedule, long nodes, int variant) {
+  if (p < 2 || schedule != SE2W_SCHED_FUSED) return true;
+  if (is_reg64_variant(variant)) return mode == SE2W_FP64 && p < 5;
+  if (is_col_variant(variant)) return mode != SE2W_FP64 || p >= 5 || nodes < 2000000;
+  return is_reg_variant(variant);
+}
+
 void reg_shape(int variant, int &tex, int &tey) {
   const RegSchedule &r = kRegSchedules[reg_schedule_of(variant)];
   tex = r.ex - 1;
@@ -347,6 +372,11 @@ void set_tiling(se2w_ctx *c) {
     c->tex = kReg64Schedules[c->variant - SE2W_KERNEL_REG64].ex - 1;
     c->tey = kReg64Schedules[c->variant - SE2W_KERNEL_REG64].ey - 1;
   }
+  else if (is_col_variant(c->variant)) {
+    const ColSchedule &r = kColSchedules[c->variant - SE2W_KERNEL_COL];
+    c->tex = r.wx * col_epw(c->p) - 1;
+    c->tey = r.ey - 1;
+  }
   else if (c->variant == SE2W_KERNEL_MFMA || c->variant == SE2W_KERNEL_LINE) mfma_shape(c->p, c->tex, c->tey);
   else tile_shape(c->p, c->mode, c->tex, c->tey);
   c->tiles_x = (c->mx + c->tex - 1) / c->tex;
@@ -380,6 +410,7 @@ StepParams<typename RealOf<MODE>::T> make_params(se2w_ctx *c, int step, double d
   p.elem_dy = (const R *)c->edy;
   p.D = (const R *)c->D;
   p.w2 = (const R *)c->w2;
+  p.dny = (const R *)c->dny;
   p.tile_src_ptr = c->d_tsrc_ptr; p.tile_src_idx = c->d_tsrc_idx; p.src_elem = c->d_src_elem;
   p.src_vals = (const R *)c->d_src_vals; p.psi = (const R *)c->d_psi; p.ns = c->ns;
   p.tile_rec_ptr = c->d_trec_ptr; p.tile_rec_idx = c->d_trec_idx; p.rec_elem = c->d_rec_elem;
@@ -698,7 +729,7 @@ int se2w_destroy(se2w_ctx *c) {
   if (c->stream) hipStreamSynchronize(c->stream);
   if (c->C[1] == c->C[0]) c->C[1] = nullptr;  // aliased compensation buffer
   void **bufs[] = {&c->U[0], &c->U[1], &c->C[0], &c->C[1], &c->V, &c->A, &c->Vn, &c->Cn, &c->F, &c->Utmp, &c->mass, &c->lambda,
-                   &c->mu, &c->edx, &c->edy, &c->D, &c->w2, &c->d_src_vals, &c->d_psi, &c->d_rec, &c->d_erec};
+                   &c->mu, &c->edx, &c->edy, &c->D, &c->w2, &c->dny, &c->d_src_vals, &c->d_psi, &c->d_rec, &c->d_erec};
   for (void **b : bufs) dev_free(*b);
   int **ibufs[] = {&c->d_src_elem, &c->d_tsrc_ptr, &c->d_tsrc_idx, &c->d_rec_elem, &c->d_rec_gll,
                     &c->d_trec_ptr, &c->d_trec_idx, &c->d_erec_elem, &c->d_terec_ptr, &c->d_terec_idx};
@@ -734,10 +765,21 @@ int se2w_set_tables(se2w_ctx *c, const double *D, const double *w1d, const doubl
   std::vector<double> w2((size_t)nb * nb);
   for (int j = 0; j < nb; j++)
     for (int i = 0; i < nb; i++) w2[i + j * nb] = w1d[i] * w1d[j];  // se2wave.c:860-865
+  std::vector<double> dd((size_t)2 * nb * nb);  // D and its transpose
+  for (int q = 0; q < nb; q++)
+    for (int i = 0; i < nb; i++) dd[(size_t)q * nb + i] = dd[(size_t)nb * nb + i * nb + q] = D[q * nb + i];
   int ierr;
-  if ((ierr = upload_real(c, &c->D, D, (size_t)nb * nb)) || (ierr = upload_real(c, &c->w2, w2.data(), w2.size())) ||
+  if ((ierr = upload_real(c, &c->D, dd.data(), dd.size())) || (ierr = upload_real(c, &c->w2, w2.data(), w2.size())) ||
       (ierr = upload_real(c, &c->edx, elem_dx, c->mx)) || (ierr = upload_real(c, &c->edy, elem_dy, c->my)))
     return ierr;
+  if (c->mode == SE2W_FP64) {  // dN_dy of each element row, rounded as in se2wave.c:1276
+    std::vector<double> dny((size_t)c->my * nb * nb);
+    for (int e = 0; e < c->my; e++) {
+      const double iJ11 = 1.0 / (0.5 * elem_dy[e]);
+      for (int k = 0; k < nb * nb; k++) dny[(size_t)e * nb * nb + k] = iJ11 * D[k];
+    }
+    if ((ierr = upload<double>(&c->dny, dny.data(), dny.size(), c->stream))) return ierr;
+  }
   c->hD.assign(D, D + (size_t)nb * nb);
   c->hdx.assign(elem_dx, elem_dx + c->mx);
   c->hdy.assign(elem_dy, elem_dy + c->my);
@@ -1289,7 +1331,8 @@ int se2w_get_timing(se2w_ctx *c, double *run_ms, double kernel_ms[2]) {
 int se2w_set_kernel(se2w_ctx *c, int32_t variant) {
   if (!c) return fail(SE2W_ERR_ARG, "null context");
   if (variant != SE2W_KERNEL_LDS && !is_reg_variant(variant) && variant != SE2W_KERNEL_MFMA &&
-      variant != SE2W_KERNEL_LINE && variant != SE2W_KERNEL_LDS_WIDE && !is_reg64_variant(variant))
+      variant != SE2W_KERNEL_LINE && variant != SE2W_KERNEL_LDS_WIDE && !is_reg64_variant(variant) &&
+      !is_col_variant(variant))
     return fail(SE2W_ERR_ARG, "unknown kernel %d", variant);
   if (is_reg64_variant(variant) && !reg64_variant_built(c->p, c->mode, variant, c->schedule))
     return fail(SE2W_ERR_UNSUPPORTED,
@@ -1303,6 +1346,9 @@ int se2w_set_kernel(se2w_ctx *c, int32_t variant) {
     return fail(SE2W_ERR_UNSUPPORTED, "matrix-core kernel needs FP32, 6 <= p <= 8 and the fused schedule");
   if (variant == SE2W_KERNEL_LINE && !mfma_available(c->p, c->mode, c->schedule))
     return fail(SE2W_ERR_UNSUPPORTED, "line kernel needs FP32, 6 <= p <= 8 and the fused schedule");
+  if (is_col_variant(variant) && !col_variant_built(c->p, c->mode, variant, c->schedule))
+    return fail(SE2W_ERR_UNSUPPORTED,
+                "the column kernel needs 2 <= p <= %d and the fused schedule (in FP64 its first form only)", kMaxP);
   if (is_reg_variant(variant) && !reg_available(c->p, c->mode))
     return fail(SE2W_ERR_UNSUPPORTED, "register-blocked kernel needs FP32 and 2 <= p <= 8");
   if (is_reg_variant(variant) && !reg_variant_built(c->p, variant, c->schedule))
@@ -1328,7 +1374,7 @@ int se2w_set_kernel(se2w_ctx *c, int32_t variant) {
   return SE2W_OK;
 }
 
-int se2w_kernel_count(void) { return SE2W_KERNEL_REG64 + kNumReg64Schedules; }
+int se2w_kernel_count(void) { return kNumVariants; }
 
 // Autotuner: times every variant built for the context's (p, precision,
 // schedule) on the context's own mesh and keeps the fastest.  The state is
@@ -1414,10 +1460,15 @@ int se2w_autotune(se2w_ctx *c, int32_t steps, int32_t reps, int32_t *best_varian
       if (reg_variant_built(c->p, SE2W_KERNEL_REG + k, c->schedule)) cands.push_back(SE2W_KERNEL_REG + k);
   for (int k = 0; k < kNumReg64Schedules; k++)
     if (reg64_variant_built(c->p, c->mode, SE2W_KERNEL_REG64 + k, c->schedule)) cands.push_back(SE2W_KERNEL_REG64 + k);
+  for (int v = SE2W_KERNEL_COL; v < kNumVariants; v++)
+    if (col_variant_built(c->p, c->mode, v, c->schedule)) cands.push_back(v);
   if (mfma_available(c->p, c->mode, c->schedule)) {
     cands.push_back(SE2W_KERNEL_MFMA);
     cands.push_back(SE2W_KERNEL_LINE);
   }
+  cands.erase(std::remove_if(cands.begin(), cands.end(),
+                             [&](int v) { return !tuning_candidate(c->p, c->mode, c->schedule, (long)c->nx * c->ny, v); }),
+              cands.end());
   Snapshot sn;
   if (int ierr = snapshot_take(c, sn)) return ierr;
   const int variant0 = c->variant;
@@ -1686,8 +1737,10 @@ int se2w_ensemble_autotune(se2w_ensemble *e, int32_t steps, int32_t reps, int32_
   if (!e || steps < 1 || reps < 1) return fail(SE2W_ERR_ARG, "bad autotune arguments");
   HIPCHK(hipSetDevice(e->device));
   std::vector<int> cands;
-  for (int v = 0; v < SE2W_KERNEL_REG64 + kNumReg64Schedules; v++)
-    if (ens_variant_built(e, v)) cands.push_back(v);
+  long nodes = 0;
+  for (const se2w_ctx *c : e->members) nodes += (long)c->nx * c->ny;
+  for (int v = 0; v < kNumVariants; v++)
+    if (ens_variant_built(e, v) && tuning_candidate(e->p, e->mode, SE2W_SCHED_FUSED, nodes, v)) cands.push_back(v);
   const size_t n = e->members.size();
   std::vector<Snapshot> sn(n);
   for (size_t i = 0; i < n; i++) {

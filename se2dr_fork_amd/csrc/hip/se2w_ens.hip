@@ -5,6 +5,7 @@
 #include "se2w_ens.hpp"
 
 #include "se2w.h"
+#include "se2w_kernels_col.hpp"
 #include "se2w_kernels_reg.hpp"
 #include "se2w_kernels_reg64.hpp"
 #include "se2w_kernels_mfma.hpp"
@@ -70,6 +71,12 @@ void ens_reg64_kernel(EnsArgs<double> a) {
   });
 }
 
+template <int P, int MODE, int WX, int EY>
+__global__ __launch_bounds__(64 * WX * EY) __attribute__((amdgpu_waves_per_eu(col_waves(P, MODE), 8)))
+void ens_col_kernel(EnsArgs<typename RealOf<MODE>::T> a) {
+  ens_tile(a, [](auto &prm, int tile, int step, int last) { col_body<P, MODE, WX, EY>(prm, tile, step, last); });
+}
+
 template <int P, int MODE>
 __global__ __launch_bounds__(kThreads) void ens_mfma_kernel(EnsArgs<float> a) {
   ens_tile(a, [](auto &prm, int tile, int step, int last) { mfma_body<P, MODE, false>(prm, tile, step, last); });
@@ -130,6 +137,30 @@ int reg64_dispatch(int sched, const void *args, int grid, hipStream_t s, int *bp
   return -1;
 }
 
+template <int P, int MODE, int S>
+int col_dispatch(int sched, const void *args, int grid, hipStream_t s, int *bpc, int *thr) {
+  if constexpr (S < kNumColSchedules) {
+    if constexpr (col_schedule_built(P, MODE, S, true)) {
+      if (sched == S) {
+        constexpr ColSchedule r = kColSchedules[S];
+        auto k = ens_col_kernel<P, MODE, r.wx, r.ey>;
+        const int nt = 64 * r.wx * r.ey;
+        if (!args) {
+          int n = 0;
+          if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, nt, 0) != hipSuccess) return -1;
+          *bpc = n;
+          *thr = nt;
+          return 0;
+        }
+        hipLaunchKernelGGL(k, dim3(grid), dim3(nt), 0, s, *(const EnsArgs<typename RealOf<MODE>::T> *)args);
+        return 0;
+      }
+    }
+    return col_dispatch<P, MODE, S + 1>(sched, args, grid, s, bpc, thr);
+  }
+  return -1;
+}
+
 template <int P, int MODE>
 int dispatch_pm(int variant, const void *args, int grid, hipStream_t s, int *bpc, int *thr) {
   using R = typename RealOf<MODE>::T;
@@ -159,6 +190,10 @@ int dispatch_pm(int variant, const void *args, int grid, hipStream_t s, int *bpc
       hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, s, *(const EnsArgs<float> *)args);
       return 0;
     }
+  }
+  if constexpr (P >= 2) {
+    if (variant >= SE2W_KERNEL_COL)
+      return col_dispatch<P, MODE, 0>(variant - SE2W_KERNEL_COL, args, grid, s, bpc, thr);
   }
   if constexpr (MODE != MODE_F64 && P >= 2)
     return reg_dispatch<P, MODE, 0>(variant - SE2W_KERNEL_REG, args, grid, s, bpc, thr);

@@ -77,8 +77,9 @@ template <typename R> struct StepParams {
   const R *mass;   // MODE_F64: lumped mass M; FP32 modes: 1/M (per node, padded)
   const R *lambda, *mu;
   const R *elem_dx, *elem_dy;
-  const R *D;      // D[q*(P+1) + i] = dN_i/dxi at GLL node q
+  const R *D;      // D[q*(P+1) + i] = dN_i/dxi at GLL node q; then its transpose
   const R *w2;     // w2[i + j*(P+1)] = w_i * w_j
+  const R *dny;    // MODE_F64: dny[ej][q*(P+1) + i] = D[q*(P+1) + i] / J11 of element row ej
   // sources (CSR per tile)
   const int *tile_src_ptr, *tile_src_idx, *src_elem;
   const R *src_vals;  // [ns][2*npe]

@@ -16,7 +16,14 @@
 // kernels) holds 2 (p+1)^2 values per component, which takes a SIMD's whole
 // register file in FP64 (one wave, scratch traffic from p = 7 on), and small
 // meshes give such a kernel too few waves.  Here a lane holds a few times
-// p + 1 values, and a mesh gives (p+1)/2 times the waves.
+// p + 1 values (three waves per SIMD in FP64, four in FP32), and a mesh gives
+// (p+1)/2 times the waves.  It is bound by VALU issue and by the latency of
+// its phases.  us per step, fastest register or LDS kernel -> this one: FP64
+// 24^2 p4 15.0 -> 9.2, 256^2 p4 26.1 -> 22.6, 800^2 p4 189 -> 211, 389^2 p5
+// 93 -> 69, 64^2 p6 21.9 -> 12.0, 330^2 p6 152 -> 86, 300^2 p7 297 -> 97,
+// 256^2 p8 239 -> 107; FP32 512^2 p4 32.0 -> 33.8, 320^2 p5 28.3 -> 23.2,
+// 200^2 p6 24.0 -> 18.3, 500^2 p6 74 -> 72, 300^2 p7 51 -> 36, 512^2 p8 198 ->
+// 166; FP32+Kahan 512^2 p8 259 -> 225.
 //
 // Every sum runs over the same terms in the same order, with the same
 // roundings, as in reg64_body / reg_body, so the results have the same bits
@@ -36,13 +43,19 @@
 
 namespace se2w {
 
-// Schedules: waves in x, element rows, minimum waves per SIMD.
-struct ColSchedule { int wx, ey, waves; };
-constexpr ColSchedule kColSchedules[] = {{1, 4, 3}, {1, 8, 3}};
+// Schedules: waves in x, element rows.  Four rows (of which three are owned)
+// leave the most workgroups per CU and are the fastest in FP64 at every degree
+// and size (7 % ahead of eight rows at 256 x 256 p8, level at 330 x 330 p6);
+// FP32 needs half the registers and LDS, and eight rows, seven of them owned,
+// are ahead by up to 5 % on some large meshes (512 x 512 p8: 166 against 172).  Two waves in x and six rows measured
+// slower than either (64 x 64 p6 FP64: 12.0, 15.8, 13.9 and 15.1 us for 1 x 4,
+// 1 x 8, 2 x 4 and 1 x 6).
+struct ColSchedule { int wx, ey; };
+constexpr ColSchedule kColSchedules[] = {{1, 4}, {1, 8}};
 constexpr int kNumColSchedules = sizeof(kColSchedules) / sizeof(kColSchedules[0]);
 constexpr int col_epw(int p) { return 64 / (p + 1); }  // elements per wave
-constexpr bool col_schedule_built(int P, int S, bool fused) {
-  return fused && P >= 2 && P <= kMaxP && S >= 0 && S < kNumColSchedules;
+constexpr bool col_schedule_built(int P, int mode, int S, bool fused) {
+  return fused && P >= 2 && P <= kMaxP && S >= 0 && S < (mode == MODE_F64 ? 1 : kNumColSchedules);
 }
 
 // Orders the LDS accesses of one wave: its LDS instructions execute in order,
@@ -50,6 +63,15 @@ constexpr bool col_schedule_built(int P, int S, bool fused) {
 __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
+}
+
+// The same uniform pointer, opaque to the compiler: a table read through it is
+// loaded where it is used.  Hoisted out of the row loops the tables take more
+// SGPRs than there are, and every use of a spilled one costs a VALU move.
+template <typename T>
+__device__ __forceinline__ T *here(T *p) {
+  asm volatile("" : "+s"(p));
+  return p;
 }
 
 template <int P, int MODE, int WX, int EY, typename PRM>
@@ -78,6 +100,31 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
   const bool owner = row_valid && ly >= 1 && lx >= 1 && ex < ex_end && lane < EPW * NB;
   R2 *B = &buf[ly][lx][0];  // [j][i]
 
+  // The update's loads.  Nodes that the lane does not own load an owned node
+  // instead (in bounds, unused), so they carry no branch.  Where the registers
+  // allow they go out between the two halves of the element operator, in place
+  // of the displacement column, and the forces cover their latency (EARLY);
+  // else before the barrier.
+  constexpr bool EARLY = MODE != MODE_F64;
+  const bool rb = ex == prm.mx - 1, tb = ey == prm.my - 1;  // domain right / top boundary
+  const bool mine = owner && (i < P || rb);
+  const int gx = mine ? ex * P + i : ex0 * P;
+  const int gy0 = mine ? ey * P : ey0 * P;
+  const long idx0 = (long)gy0 * prm.pitch + gx;
+  R2 pu[NB], pv[NB], pc[NB];
+  R pm[NB];
+  auto node_loads = [&]() {
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+      const long idx = idx0 + (long)(j < P || (mine && tb) ? j : 0) * prm.pitch;
+      pu[j] = prm.u_in[idx];
+      pv[j] = prm.v[idx];
+      pm[j] = prm.mass[idx];
+      if constexpr (MODE == MODE_F32K) pc[j] = prm.c_in[idx];
+      else pc[j] = R2{R(0), R(0)};
+    }
+  };
+
   R2 F[NB];  // forces of the nodes (i, j)
   if (row_valid) {
     // columns of elements outside the mesh repeat its first or last column of
@@ -96,14 +143,20 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
 #pragma unroll
     for (int j = 0; j < NB; j++) B[j * NB + i] = u[j];
     // derivatives along a row: at the lane's points dr[k] (of node column k),
-    // at the lane's nodes dc[k] (from point column k)
+    // at the lane's nodes dc[k] (from point column k, a row of D's transpose);
+    // weights of the lane's points (the table is symmetric).  Rows, so that a
+    // lane's values come in few wide loads.
     R dr[NB], dc[NB], w[NB];
+    auto load_force_tables = [&]() {
 #pragma unroll
-    for (int k = 0; k < NB; k++) {
-      dr[k] = prm.D[i * NB + k];
-      dc[k] = prm.D[k * NB + i];
-      w[k] = prm.w2[i + k * NB];
-    }
+      for (int k = 0; k < NB; k++) {
+        dc[k] = prm.D[NB * NB + i * NB + k];
+        w[k] = prm.w2[i * NB + k];
+      }
+    };
+#pragma unroll
+    for (int k = 0; k < NB; k++) dr[k] = prm.D[i * NB + k];
+    if constexpr (MODE != MODE_F64) load_force_tables();
     wave_lds_order();
     if constexpr (MODE == MODE_F64) {
       // dN_dy of the element row, iJ11 D[qj][j], formed once on the host
@@ -112,20 +165,20 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
 #pragma unroll
       for (int k = 0; k < NB; k++) {
         dr[k] = iJ00 * dr[k];
-        dc[k] = iJ00 * dc[k];
         own[k] = k == i ? R(1) : R(0);
       }
       R sxx[NB], sxy[NB], syy[NB];
 #pragma unroll
       for (int qj = 0; qj < NB; qj++) {
+        CR *dq = here(dny + qj * NB);
         R e0 = R(0), e1 = R(0), e2 = R(0);
 #pragma unroll
         for (int j = 0; j < qj; j++) {
-          e1 = e1 + dny[qj * NB + j] * u[j].y;
-          e2 = e2 + dny[qj * NB + j] * u[j].x;
+          e1 = e1 + dq[j] * u[j].y;
+          e2 = e2 + dq[j] * u[j].x;
         }
-        e1 = e1 + dny[qj * NB + qj] * u[qj].y;
-        const R tq = dny[qj * NB + qj] * u[qj].x;
+        e1 = e1 + dq[qj] * u[qj].y;
+        const R tq = dq[qj] * u[qj].x;
 #pragma unroll
         for (int k = 0; k < NB; k++) {
           const R2 uk = B[qj * NB + k];
@@ -134,73 +187,85 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
         }
 #pragma unroll
         for (int j = qj + 1; j < NB; j++) {
-          e1 = e1 + dny[qj * NB + j] * u[j].y;
-          e2 = e2 + dny[qj * NB + j] * u[j].x;
+          e1 = e1 + dq[j] * u[j].y;
+          e2 = e2 + dq[j] * u[j].x;
         }
         sxx[qj] = c11 * e0 + lam * e1;
         syy[qj] = lam * e0 + c11 * e1;
         sxy[qj] = mu * e2;
       }
+      // after the displacement's last use: the registers take the one or the
+      // other
       wave_lds_order();
+      load_force_tables();
+#pragma unroll
+      for (int k = 0; k < NB; k++) dc[k] = iJ00 * dc[k];
+      if constexpr (EARLY) node_loads();
 #pragma unroll
       for (int qj = 0; qj < NB; qj++) B[qj * NB + i] = R2{sxx[qj], sxy[qj]};
       wave_lds_order();
       // row terms of node row j: points (k, j), k ascending, the lane's own
       // point with its column term inside
-      auto row_terms = [&](int j, R2 &f) {
-        const R cx = dny[j * NB + j] * sxy[j], cy = dny[j * NB + j] * syy[j];
+      auto row_terms = [&](int j, CR *dq, R2 &f) {
+        const R cx = dq[j] * sxy[j], cy = dq[j] * syy[j];
+        CR *wq = here(W + j * NB);
 #pragma unroll
         for (int k = 0; k < NB; k++) {
           const R2 s = B[j * NB + k];
-          const R nfac = -(detJ * W[k + j * NB]);
+          const R nfac = -(detJ * wq[k]);
           f.x = f.x + nfac * fma(own[k], cx, dc[k] * s.x);
           f.y = f.y + nfac * fma(own[k], cy, dc[k] * s.y);
         }
       };
-      auto column_term = [&](int qj, int j, R2 &f) {
+      auto column_term = [&](int qj, int j, CR *dq, R2 &f) {
         const R nfac = -(detJ * w[qj]);
-        f.x = f.x + nfac * (dny[qj * NB + j] * sxy[qj]);
-        f.y = f.y + nfac * (dny[qj * NB + j] * syy[qj]);
+        f.x = f.x + nfac * (dq[j] * sxy[qj]);
+        f.y = f.y + nfac * (dq[j] * syy[qj]);
       };
       if (ly == 0) {  // uniform per wave
         R2 f = R2{R(0), R(0)};
 #pragma unroll
-        for (int qj = 0; qj < P; qj++) column_term(qj, P, f);
-        row_terms(P, f);
+        for (int qj = 0; qj < P; qj++) column_term(qj, P, dny + qj * NB, f);
+        row_terms(P, dny + P * NB, f);
         F[P] = f;
       } else {
 #pragma unroll
         for (int j = 0; j < NB; j++) F[j] = R2{R(0), R(0)};
 #pragma unroll
         for (int qj = 0; qj < NB; qj++) {
-          row_terms(qj, F[qj]);
+          CR *dq = here(dny + qj * NB);
+          row_terms(qj, dq, F[qj]);
 #pragma unroll
           for (int j = 0; j < NB; j++)
-            if (j != qj) column_term(qj, j, F[j]);
+            if (j != qj) column_term(qj, j, dq, F[j]);
         }
       }
     } else {
       const R s = -detJ;
       const R a1 = s * c11 * iJ00 * iJ00, a2 = s * lam * iJ00 * iJ11, a3 = s * c11 * iJ11 * iJ11;
       const R b1 = s * mu * iJ11 * iJ11, b2 = s * mu * iJ00 * iJ11, b3 = s * mu * iJ00 * iJ00;
+      // rows of D, held in SGPRs up to p = 6
+      auto table_row = [&](int qj) { return P > 6 ? here(D + qj * NB) : D + qj * NB; };
       // row stresses (A, Cx) and column stresses (Bs, E), as in
       // RegOperator::row_stress
       R2 rs[NB], cs[NB];
 #pragma unroll
       for (int qj = 0; qj < NB; qj++) {
+        CR *dq = table_row(qj);
         R dxux = R(0), dxuy = R(0), dyux = R(0), dyuy = R(0);
 #pragma unroll
         for (int k = 0; k < NB; k++) {
           const R2 uk = B[qj * NB + k];
           dxux = fma(dr[k], uk.x, dxux);
           dxuy = fma(dr[k], uk.y, dxuy);
-          dyux = fma((R)D[qj * NB + k], u[k].x, dyux);
-          dyuy = fma((R)D[qj * NB + k], u[k].y, dyuy);
+          dyux = fma((R)dq[k], u[k].x, dyux);
+          dyuy = fma((R)dq[k], u[k].y, dyuy);
         }
         rs[qj] = R2{w[qj] * fma(a1, dxux, a2 * dyuy), w[qj] * fma(b3, dxuy, b2 * dyux)};
         cs[qj] = R2{w[qj] * fma(b1, dyux, b2 * dxuy), w[qj] * fma(a3, dyuy, a2 * dxux)};
       }
       wave_lds_order();
+      node_loads();
 #pragma unroll
       for (int qj = 0; qj < NB; qj++) B[qj * NB + i] = rs[qj];
       wave_lds_order();
@@ -212,25 +277,26 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
           f.y = fma(dc[k], t.y, f.y);
         }
       };
-      auto column_term = [&](int qj, int j, R2 &f) {
-        f.x = fma((R)D[qj * NB + j], cs[qj].x, f.x);
-        f.y = fma((R)D[qj * NB + j], cs[qj].y, f.y);
+      auto column_term = [&](int qj, int j, CR *dq, R2 &f) {
+        f.x = fma((R)dq[j], cs[qj].x, f.x);
+        f.y = fma((R)dq[j], cs[qj].y, f.y);
       };
       if (ly == 0) {
         R2 f = R2{R(0), R(0)};
 #pragma unroll
-        for (int qj = 0; qj < P; qj++) column_term(qj, P, f);
+        for (int qj = 0; qj < P; qj++) column_term(qj, P, D + qj * NB, f);
         row_terms(P, f);
-        column_term(P, P, f);
+        column_term(P, P, D + P * NB, f);
         F[P] = f;
       } else {
 #pragma unroll
         for (int j = 0; j < NB; j++) F[j] = R2{R(0), R(0)};
 #pragma unroll
         for (int qj = 0; qj < NB; qj++) {
+          CR *dq = table_row(qj);
           row_terms(qj, F[qj]);
 #pragma unroll
-          for (int j = 0; j < NB; j++) column_term(qj, j, F[j]);
+          for (int j = 0; j < NB; j++) column_term(qj, j, dq, F[j]);
         }
       }
     }
@@ -244,53 +310,47 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
     }
     B[P * NB + i] = F[P];
   }
-  // The update's loads go out before the barrier; nodes that the lane does
-  // not own load an owned node instead (in bounds, unused), so they carry no
-  // branch.
-  const bool rb = ex == prm.mx - 1, tb = ey == prm.my - 1;  // domain right / top boundary
-  const bool mine = owner && (i < P || rb);
-  const int gx = mine ? ex * P + i : ex0 * P;
-  const int gy0 = mine ? ey * P : ey0 * P;
-  const long idx0 = (long)gy0 * prm.pitch + gx;
-  R2 pu[NB], pv[NB], pc[NB];
-  R pm[NB];
-#pragma unroll
-  for (int j = 0; j < NB; j++) {
-    const long idx = idx0 + (long)(j < P || (mine && tb) ? j : 0) * prm.pitch;
-    pu[j] = prm.u_in[idx];
-    pv[j] = prm.v[idx];
-    pm[j] = prm.mass[idx];
-    if constexpr (MODE == MODE_F32K) pc[j] = prm.c_in[idx];
-    else pc[j] = R2{R(0), R(0)};
-  }
+  if constexpr (!EARLY) node_loads();
   const TileLists tl = tile_lists(prm, tile, step, last);
   __syncthreads();
   if (!mine) return;
   const bool left = ex > 0 && i == 0, below = ey > 0;
   // the own force and the neighbours' in ascending element order
   const R2 *L = &buf[ly][lx - 1][0], *Dn = &buf[ly - 1][lx][0], *Dg = &buf[ly - 1][lx - 1][0];
+  auto update = [&](const TileLists &t) {
 #pragma unroll
-  for (int j = 0; j < NB; j++) {
-    if (j == P && !tb) break;
-    R2 g = F[j];
-    if (j == 0 && below) {
-      R2 t = Dn[P * NB + i];
-      if (left) {  // (ex-1,ey-1), (ex,ey-1), (ex-1,ey), own
-        const R2 d = Dg[P * NB + P], l = L[P];
-        t = R2{(d.x + t.x) + l.x, (d.y + t.y) + l.y};
+    for (int j = 0; j < NB; j++) {
+      if (j < P || tb) {
+        R2 g = F[j];
+        if (j == 0 && below) {
+          R2 f = Dn[P * NB + i];
+          if (left) {  // (ex-1,ey-1), (ex,ey-1), (ex-1,ey), own
+            const R2 d = Dg[P * NB + P], l = L[P];
+            f = R2{(d.x + f.x) + l.x, (d.y + f.y) + l.y};
+          }
+          g = R2{f.x + g.x, f.y + g.y};
+        } else if (left) {
+          const R2 l = L[j * NB + P];
+          g = R2{l.x + g.x, l.y + g.y};
+        }
+        node_update_core<P, MODE>(prm, t, gx, gy0 + j, idx0 + (long)j * prm.pitch, g.x, g.y, pu[j].x, pu[j].y, pv[j],
+                                  pm[j], pc[j]);
       }
-      g = R2{t.x + g.x, t.y + g.y};
-    } else if (left) {
-      const R2 l = L[j * NB + P];
-      g = R2{l.x + g.x, l.y + g.y};
     }
-    node_update_core<P, MODE>(prm, tl, gx, gy0 + j, idx0 + (long)j * prm.pitch, g.x, g.y, pu[j].x, pu[j].y, pv[j],
-                              pm[j], pc[j]);
-  }
+  };
+  // Almost every tile and step has no source, no receiver and no last-step
+  // stores: a copy of the update without them, p + 1 nodes of straight code.
+  if (tl.empty() && !last) update(TileLists{0, 0, 0, 0, 0, 0, step, 0});
+  else update(tl);
 }
 
-template <int P, int MODE, int WX, int EY, int WAVES>
-__global__ __launch_bounds__(64 * WX * EY) __attribute__((amdgpu_waves_per_eu(WAVES, 8)))
+// Minimum waves per SIMD, i.e. the registers per lane.
+constexpr int col_waves(int p, int mode) {
+  return mode == MODE_F64 ? (p <= 4 ? 4 : p <= 7 ? 3 : 2) : mode == MODE_F32K && p == 8 ? 3 : 4;
+}
+
+template <int P, int MODE, int WX, int EY>
+__global__ __launch_bounds__(64 * WX * EY) __attribute__((amdgpu_waves_per_eu(col_waves(P, MODE), 8)))
 void col_kernel(StepParams<typename RealOf<MODE>::T> prm) {
   const int tile = tile_of_block(blockIdx.x, prm.tiles_per_xcd);
   if (tile >= prm.tiles_x * prm.tiles_y) return;  // uniform per workgroup

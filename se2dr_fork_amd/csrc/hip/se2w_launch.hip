@@ -4,6 +4,7 @@
 #include "se2w_launch.hpp"
 
 #include "se2w.h"
+#include "se2w_kernels_col.hpp"
 #include "se2w_kernels_mfma.hpp"
 #include "se2w_kernels_reg.hpp"
 #include "se2w_kernels_reg64.hpp"
@@ -36,6 +37,22 @@ bool launch_reg64_s(const LaunchCfg &c, const StepParams<R> &prm) {
   return false;
 }
 
+template <int P, int S>
+bool launch_col_s(const LaunchCfg &c, const StepParams<R> &prm) {
+  if constexpr (S < kNumColSchedules) {
+    if constexpr (col_schedule_built(P, kMode, S, true)) {
+      if (c.variant - SE2W_KERNEL_COL == S) {
+        constexpr ColSchedule r = kColSchedules[S];
+        hipLaunchKernelGGL((col_kernel<P, kMode, r.wx, r.ey>), dim3(c.grid), dim3(64 * r.wx * r.ey), 0, c.stream,
+                           prm);
+        return true;
+      }
+    }
+    return launch_col_s<P, S + 1>(c, prm);
+  }
+  return false;
+}
+
 template <int P, bool FUSED, int S>
 bool launch_reg_s(const LaunchCfg &c, const StepParams<R> &prm) {
   if constexpr (kMode != MODE_F64 && S < kNumRegSchedules) {
@@ -58,6 +75,9 @@ bool launch_reg_s(const LaunchCfg &c, const StepParams<R> &prm) {
 template <int P, bool FUSED>
 void launch_element_p(const LaunchCfg &c, const StepParams<R> &prm) {
   const dim3 grid(c.grid);
+  if constexpr (FUSED && P >= 2) {
+    if (c.variant >= SE2W_KERNEL_COL && launch_col_s<P, 0>(c, prm)) return;
+  }
   if constexpr (kMode != MODE_F64 && P >= 2) {
     if (is_reg(c.variant) && launch_reg_s<P, FUSED, 0>(c, prm)) return;
   }

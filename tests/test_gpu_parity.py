@@ -689,3 +689,30 @@ def test_wide_tile_kernel_equals_the_tile_kernel(p):
             np.testing.assert_array_equal(u1, u0)
             np.testing.assert_array_equal(v1, v0)
             np.testing.assert_array_equal(a1, a0)
+
+
+@pytest.mark.parametrize("p", range(2, 9))
+@pytest.mark.parametrize("mx, my", [(1, 1), (2, 9), (23, 4), (41, 15)])
+def test_column_kernel_has_the_other_kernels_bits(oracle, p, mx, my):
+    """One lane per element column: FP64 bit-identical to the oracle, the FP32
+    modes to the register kernel, on one element, one or two columns of tiles,
+    one tile row and partial edge tiles at every degree (tiles of 63 // (p+1)
+    elements), with sources and receivers on shared nodes."""
+    hip, _ = S.libraries()
+    variants = range(S.KERNEL_COL, hip.se2w_kernel_count())  # FP64 has the first
+    sc = SC.small(mx=mx, my=my, p=p, nt=24, seed=300 + p + mx, nsrc=3, nrec=7)
+    sc.use_nearest_internal_gll = p > 1
+    b0 = SC.build(sc, with_solver=False)
+    _, ro, uo, vo, ao = oracle.Problem(sc, dt=b0.dt, nt=b0.nsteps).run()
+    for k in variants[:1]:
+        b, _, rows, u, v, a = gpu_run(sc, kernel=k, chunks=2)
+        for got, want in ((rows, ro), (u, uo), (v, vo), (a, ao)):
+            np.testing.assert_array_equal(got, want, err_msg=f"variant {k}")
+        b.solver.close()
+    reg = S.KERNEL_REG if p < 7 else S.KERNEL_REG + 3
+    for prec in (S.FP32, S.FP32_KAHAN):
+        want = gpu_run(sc, precision=prec, kernel=reg, chunks=2)
+        for k in variants:
+            got = gpu_run(sc, precision=prec, kernel=k, chunks=2)
+            for x, y in zip(got[2:], want[2:]):
+                np.testing.assert_array_equal(x, y, err_msg=f"variant {k} precision {prec}")

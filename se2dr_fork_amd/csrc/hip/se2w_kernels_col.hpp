@@ -21,9 +21,9 @@
 // its phases.  us per step, fastest register or LDS kernel -> this one: FP64
 // 24^2 p4 15.0 -> 9.2, 256^2 p4 26.1 -> 22.6, 800^2 p4 189 -> 211, 389^2 p5
 // 93 -> 69, 64^2 p6 21.9 -> 12.0, 330^2 p6 152 -> 86, 300^2 p7 297 -> 97,
-// 256^2 p8 239 -> 107; FP32 512^2 p4 32.0 -> 33.8, 320^2 p5 28.3 -> 23.2,
-// 200^2 p6 24.0 -> 18.3, 500^2 p6 74 -> 72, 300^2 p7 51 -> 36, 512^2 p8 198 ->
-// 166; FP32+Kahan 512^2 p8 259 -> 225.
+// 256^2 p8 239 -> 104; FP32 512^2 p4 32.0 -> 33.5, 320^2 p5 28.3 -> 23.6,
+// 200^2 p6 24.0 -> 18.3, 500^2 p6 74 -> 74, 300^2 p7 51 -> 36, 512^2 p8 199 ->
+// 167; FP32+Kahan 512^2 p8 260 -> 230.
 //
 // Every sum runs over the same terms in the same order, with the same
 // roundings, as in reg64_body / reg_body, so the results have the same bits
@@ -72,6 +72,18 @@ template <typename T>
 __device__ __forceinline__ T *here(T *p) {
   asm volatile("" : "+s"(p));
   return p;
+}
+
+// The value that lane t (uniform) holds.
+__device__ __forceinline__ int lane_value(int v, int t) { return __builtin_amdgcn_readlane(v, t); }
+__device__ __forceinline__ float lane_value(float v, int t) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), t));
+}
+__device__ __forceinline__ double lane_value(double v, int t) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)b, t);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), t);
+  return __longlong_as_double((long long)hi << 32 | lo);
 }
 
 template <int P, int MODE, int WX, int EY, typename PRM>
@@ -313,35 +325,135 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
   if constexpr (!EARLY) node_loads();
   const TileLists tl = tile_lists(prm, tile, step, last);
   __syncthreads();
-  if (!mine) return;
   const bool left = ex > 0 && i == 0, below = ey > 0;
-  // the own force and the neighbours' in ascending element order
-  const R2 *L = &buf[ly][lx - 1][0], *Dn = &buf[ly - 1][lx][0], *Dg = &buf[ly - 1][lx - 1][0];
-  auto update = [&](const TileLists &t) {
+  if (mine) {  // own force and the neighbours' in ascending element order
+    const R2 *L = &buf[ly][lx - 1][0], *Dn = &buf[ly - 1][lx][0], *Dg = &buf[ly - 1][lx - 1][0];
 #pragma unroll
     for (int j = 0; j < NB; j++) {
-      if (j < P || tb) {
-        R2 g = F[j];
-        if (j == 0 && below) {
-          R2 f = Dn[P * NB + i];
-          if (left) {  // (ex-1,ey-1), (ex,ey-1), (ex-1,ey), own
-            const R2 d = Dg[P * NB + P], l = L[P];
-            f = R2{(d.x + f.x) + l.x, (d.y + f.y) + l.y};
-          }
-          g = R2{f.x + g.x, f.y + g.y};
-        } else if (left) {
-          const R2 l = L[j * NB + P];
-          g = R2{l.x + g.x, l.y + g.y};
+      if (j == 0 && below) {
+        R2 f = Dn[P * NB + i];
+        if (left) {  // (ex-1,ey-1), (ex,ey-1), (ex-1,ey), own
+          const R2 d = Dg[P * NB + P], l = L[P];
+          f = R2{(d.x + f.x) + l.x, (d.y + f.y) + l.y};
         }
-        node_update_core<P, MODE>(prm, t, gx, gy0 + j, idx0 + (long)j * prm.pitch, g.x, g.y, pu[j].x, pu[j].y, pv[j],
-                                  pm[j], pc[j]);
+        F[j] = R2{f.x + F[j].x, f.y + F[j].y};
+      } else if (left) {
+        const R2 l = L[j * NB + P];
+        F[j] = R2{l.x + F[j].x, l.y + F[j].y};
       }
     }
+  }
+  auto update_node = [&](int j, int last_step) {
+    const TileLists none{0, 0, 0, 0, 0, 0, step, last_step};
+    node_update_core<P, MODE>(prm, none, gx, gy0 + j, idx0 + (long)j * prm.pitch, F[j].x, F[j].y, pu[j].x, pu[j].y, pv[j],
+                              pm[j], pc[j]);
   };
   // Almost every tile and step has no source, no receiver and no last-step
   // stores: a copy of the update without them, p + 1 nodes of straight code.
-  if (tl.empty() && !last) update(TileLists{0, 0, 0, 0, 0, 0, step, 0});
-  else update(tl);
+  if (tl.empty() && !last) {
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+        if (j < P || tb) update_node(j, 0);
+    }
+    return;
+  }
+  // With sources and receivers: a lane holds one list entry (64 at a time) and
+  // every lane tests its node against each in turn, so the lists cost no memory
+  // latency per node (36 elements at p = 8 with 8 receivers: 29 -> 24 us a
+  // step).  The loops are uniform and every lane takes part in them.
+  // The lane's entries of the tile's source and receiver lists, with the node
+  // coordinates of their element's first node.
+  struct ListItem { int id, x, y, gll; };
+  auto list_item = [&](const int *idx, const int *elem, int t0, int t1) {
+    ListItem it{0, 0, 0, 0};
+    if (t0 + lane < t1) {
+      it.id = idx[t0 + lane];
+      const int e = elem[it.id];
+      it.x = e % prm.mx * P;
+      it.y = e / prm.mx * P;
+    }
+    return it;
+  };
+  R psi = R(0);  // the source's value at this step
+  auto source = [&](int t0) {
+    const ListItem it = list_item(prm.tile_src_idx, prm.src_elem, t0, tl.s1);
+    psi = prm.psi[(long)step * prm.ns + it.id];
+    return it;
+  };
+  auto receiver = [&](int t0) {
+    ListItem it = list_item(prm.tile_rec_idx, prm.rec_elem, t0, tl.r1);
+    it.gll = prm.rec_gll[it.id];
+    return it;
+  };
+  ListItem src{0, 0, 0, 0}, rec{0, 0, 0, 0};
+  if (tl.s0 < tl.s1) src = source(tl.s0);
+  if (tl.r0 < tl.r1) rec = receiver(tl.r0);
+#pragma unroll
+  for (int j = 0; j < NB; j++) {
+    const bool node = mine && (j < P || tb);
+    R2 sum{R(0), R(0)};
+    bool hit = false;
+    for (int t0 = tl.s0; t0 < tl.s1; t0 += 64) {
+      if (tl.s1 - tl.s0 > 64) src = source(t0);
+      const int n = min(64, tl.s1 - t0);
+      for (int t = 0; t < n; t++) {
+        const int li = gx - lane_value(src.x, t), lj = gy0 + j - lane_value(src.y, t);
+        if (node && li >= 0 && li <= P && lj >= 0 && lj <= P) {
+          const R ps = lane_value(psi, t);
+          const long k = ((long)lane_value(src.id, t) * NB * NB + li + lj * NB) * 2;
+          sum.x = sum.x + ps * prm.src_vals[k];
+          sum.y = sum.y + ps * prm.src_vals[k + 1];
+          hit = true;
+        }
+      }
+    }
+    if (hit) F[j] = R2{F[j].x + sum.x, F[j].y + sum.y};
+    // the corrected velocity and the acceleration, as the update forms them
+    // (node_finish_f64 / _f32)
+    auto corrected = [&](R2 &v, R2 &a) {
+      if constexpr (MODE == MODE_F64) {
+        a = R2{F[j].x / pm[j], F[j].y / pm[j]};
+        v = R2{pv[j].x + prm.hdt * a.x, pv[j].y + prm.hdt * a.y};
+      } else {
+        a = R2{F[j].x * pm[j], F[j].y * pm[j]};
+        v = R2{fma(prm.hdt, a.x, pv[j].x), fma(prm.hdt, a.y, pv[j].y)};
+      }
+    };
+    for (int t0 = tl.r0; t0 < tl.r1; t0 += 64) {
+      if (tl.r1 - tl.r0 > 64) rec = receiver(t0);
+      const int n = min(64, tl.r1 - t0);
+      for (int t = 0; t < n; t++) {
+        const int li = gx - lane_value(rec.x, t), lj = gy0 + j - lane_value(rec.y, t), g = lane_value(rec.gll, t);
+        const int gi = g % NB, gj = g / NB;
+        const bool on_column = li == gi && lj >= 0 && lj <= P, on_row = lj == gj && li >= 0 && li <= P;
+        if (node && (on_column || on_row)) {
+          R2 v, a;
+          corrected(v, a);
+          R *o = prm.rec + ((long)step * prm.nr + lane_value(rec.id, t)) * rec_stride(P);
+          if (on_column) o[6 + lj] = v.x;
+          if (on_row) o[6 + NB + li] = v.y;
+          if (on_column && on_row) {
+            o[0] = pu[j].x; o[1] = pu[j].y; o[2] = v.x; o[3] = v.y; o[4] = a.x; o[5] = a.y;
+          }
+        }
+      }
+    }
+    for (int t0 = tl.q0; t0 < tl.q1; t0 += 64) {  // element receivers: every node of the element
+      const ListItem er = list_item(prm.tile_erec_idx, prm.erec_elem, t0, tl.q1);
+      const int n = min(64, tl.q1 - t0);
+      for (int t = 0; t < n; t++) {
+        const int li = gx - lane_value(er.x, t), lj = gy0 + j - lane_value(er.y, t);
+        if (node && li >= 0 && li <= P && lj >= 0 && lj <= P) {
+          R2 v, a;
+          corrected(v, a);
+          R *q = prm.erec + (((long)step * prm.ner + lane_value(er.id, t)) * (NB * NB) + li + lj * NB) * 4;
+          q[0] = pu[j].x; q[1] = pu[j].y; q[2] = v.x; q[3] = v.y;
+        }
+      }
+    }
+    if (node) update_node(j, last);
+  }
 }
 
 // Minimum waves per SIMD, i.e. the registers per lane.

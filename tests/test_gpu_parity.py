@@ -716,3 +716,25 @@ def test_column_kernel_has_the_other_kernels_bits(oracle, p, mx, my):
             got = gpu_run(sc, precision=prec, kernel=k, chunks=2)
             for x, y in zip(got[2:], want[2:]):
                 np.testing.assert_array_equal(x, y, err_msg=f"variant {k} precision {prec}")
+
+
+@pytest.mark.parametrize("p, mx, my", [(2, 19, 4), (4, 9, 5), (7, 6, 3)])
+def test_column_kernel_with_long_lists_on_one_tile(oracle, p, mx, my):
+    """More than 64 sources and receivers on a tile (a wave holds 64 list
+    entries at a time), and element receivers beside them."""
+    sc = SC.small(mx=mx, my=my, p=p, nt=20, seed=7 + p, nsrc=70, nrec=150)
+    b0 = SC.build(sc, with_solver=False)
+    _, ro, uo, vo, ao = oracle.Problem(sc, dt=b0.dt, nt=b0.nsteps).run()
+    uv = []
+    for k in (S.KERNEL_LDS, S.KERNEL_COL):
+        b = SC.build(sc)
+        b.solver.ctx.set_kernel(k)
+        xr = np.random.default_rng(p).uniform(100.0, 3900.0, (70, 2))
+        b.solver.set_uv_receivers([S.ReceiverUV(b.spec, x, interpolate=True) for x in xr])
+        _, rows = b.solver.advance(b.nsteps, b.dt)
+        u, v, a = b.solver.ctx.get_state()
+        for got, want in ((rows, ro), (u, uo), (v, vo), (a, ao)):
+            np.testing.assert_array_equal(got, want, err_msg=f"variant {k}")
+        uv.append(b.solver.uv_trace(b.nsteps))
+        b.solver.close()
+    np.testing.assert_array_equal(uv[0], uv[1])

@@ -664,7 +664,15 @@ int se2w_create(const se2w_desc *desc, se2w_ctx **out) {
   c->mode = desc->precision;
   c->schedule = desc->schedule;
   c->device = desc->device;
-  c->variant = reg_available(c->p, c->mode) && reg_variant_built(c->p, SE2W_KERNEL_REG, c->schedule)
+  // Untuned contexts (small meshes, which a trial run would cost more than it
+  // saves): in FP64 the column kernel from p = 3 up, whose waves a small mesh
+  // needs (24 x 24 p4: 9.2 us a step against 21 for the first register
+  // schedule, 24 x 24 p6 15 against 47, 16 x 16 p8 16 against 78; at p = 2 the
+  // two are level), beyond the few elements of a single register-kernel tile.
+  const bool col = c->mode == SE2W_FP64 && c->p >= 3 && (long)c->mx * c->my > 32 &&
+                   col_variant_built(c->p, c->mode, SE2W_KERNEL_COL, c->schedule);
+  c->variant = col ? SE2W_KERNEL_COL
+               : reg_available(c->p, c->mode) && reg_variant_built(c->p, SE2W_KERNEL_REG, c->schedule)
                    ? SE2W_KERNEL_REG
                : reg64_variant_built(c->p, c->mode, SE2W_KERNEL_REG64, c->schedule) ? SE2W_KERNEL_REG64
                : reg64_variant_built(c->p, c->mode, SE2W_KERNEL_REG64 + kReg64FirstP8, c->schedule)

@@ -16,8 +16,8 @@
 // kernels) holds 2 (p+1)^2 values per component, which takes a SIMD's whole
 // register file in FP64 (one wave, scratch traffic from p = 7 on), and small
 // meshes give such a kernel too few waves.  Here a lane holds a few times
-// p + 1 values (three waves per SIMD in FP64, four in FP32), and a mesh gives
-// (p+1)/2 times the waves.  It is bound by VALU issue and by the latency of
+// p + 1 values (two to four waves per SIMD in FP64, four in FP32), and a mesh
+// gives (p+1)/2 times the waves.  It is bound by VALU issue and by the latency of
 // its phases.  us per step, fastest register or LDS kernel -> this one: FP64
 // 24^2 p4 15.0 -> 9.2, 256^2 p4 26.1 -> 22.6, 800^2 p4 189 -> 211, 389^2 p5
 // 93 -> 69, 64^2 p6 21.9 -> 12.0, 330^2 p6 152 -> 86, 300^2 p7 297 -> 97,
@@ -456,7 +456,11 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
   }
 }
 
-// Minimum waves per SIMD, i.e. the registers per lane.
+// Minimum waves per SIMD, i.e. the registers per lane: the most that spill at
+// most a few registers, mostly of the update with lists.  FP64 300 x 300 p7
+// takes 94-97 us at three and 100 at two, 512 x 512 p4 74 at four and 77 at
+// three; at p = 8 three waves spill 50 registers (256 x 256: 114 us, 104-107
+// at two), and FP32+Kahan p = 8 10 at four (512 x 512: 254 us, 230 at three).
 constexpr int col_waves(int p, int mode) {
   return mode == MODE_F64 ? (p <= 4 ? 4 : p <= 7 ? 3 : 2) : mode == MODE_F32K && p == 8 ? 3 : 4;
 }

@@ -310,20 +310,82 @@ bool col_variant_built(int p, int mode, int variant, int schedule) {
   return is_col_variant(variant) && col_schedule_built(p, mode, variant - SE2W_KERNEL_COL, schedule == SE2W_SCHED_FUSED);
 }
 
-// Variants that an autotuner times: those that are the fastest on some mesh.
-// The LDS kernels are behind from p = 2 on, the matrix-core and line kernels
-// everywhere, and in FP64 the register kernels from p = 5 on (the column
-// kernel is 1.4 to 3 times as fast from 24 x 24 elements to 389 x 389).  Below,
-// in FP64, the column kernel leads up to a million nodes (256 x 256 p4: 22.6
-// against 26.1 us) and trails on large meshes (800 x 800 p4: 211 against 189
-// us), where a short trial can mistake it for the faster one: two million is
-// the line.  The kernels that are left have the same bits, so a tuned run does
-// not depend on the choice.
-bool tuning_candidate(int p, int mode, int schedule, long nodes, int variant) {
+// FP64 variants that an autotuner times, all of them with the same bits: those
+// that are the fastest on some mesh.  The LDS kernels are behind from p = 2 on
+// and the register kernels from p = 5 on (the column kernel is 1.4 to 3 times
+// as fast from 24 x 24 elements to 389 x 389).  Below, the column kernel leads
+// up to a million nodes (256 x 256 p4: 22.6 against 26.1 us) and trails on
+// large meshes (800 x 800 p4: 211 against 189 us), where a short trial can
+// mistake it for the faster one: two million is the line.
+bool tuning_candidate(int p, int schedule, long nodes, int variant) {
   if (p < 2 || schedule != SE2W_SCHED_FUSED) return true;
-  if (is_reg64_variant(variant)) return mode == SE2W_FP64 && p < 5;
-  if (is_col_variant(variant)) return mode != SE2W_FP64 || p >= 5 || nodes < 2000000;
-  return is_reg_variant(variant);
+  if (is_reg64_variant(variant)) return p < 5;
+  return is_col_variant(variant) && (p >= 5 || nodes < 2000000);
+}
+
+// The fastest of `cands` by the median of its trials, -1 if none could run:
+// `rounds` passes over the list, in each of them one untimed and n timed
+// trials of every candidate.  A candidate that fails once is out.
+template <typename Select, typename Trial>
+int fastest_of(const std::vector<int> &cands, int rounds, int n, Select select, Trial trial, double *best_ms) {
+  std::vector<std::vector<double>> t(cands.size());
+  std::vector<char> failed(cands.size(), 0);
+  for (int round = 0; round < rounds; round++)
+    for (size_t i = 0; i < cands.size(); i++) {
+      if (!failed[i]) failed[i] = select(cands[i]) != SE2W_OK;
+      for (int r = 0; r <= n && !failed[i]; r++) {
+        double ms = 0.0;
+        failed[i] = trial(&ms) != SE2W_OK;
+        if (r > 0) t[i].push_back(ms);
+      }
+    }
+  int best = -1;
+  for (size_t i = 0; i < cands.size(); i++) {
+    if (failed[i] || t[i].empty()) continue;
+    std::sort(t[i].begin(), t[i].end());
+    const double med = t[i][t[i].size() / 2];
+    if (best < 0 || med < *best_ms) { *best_ms = med; best = cands[i]; }
+  }
+  return best;
+}
+
+// The tuners' choice among the built variants.
+// FP32 modes: the LDS, matrix-core and line kernels each sum in an order of
+// their own, the register and the column kernels in the same one.  So the order
+// of the sums is settled first, by one pass over the kernels other than the
+// column kernel, and the column kernel competes only where a register kernel
+// has won.  A mesh on which an LDS kernel is the fastest of those (from p = 5
+// up to one to three million nodes) keeps its bits, though the column kernel
+// would be faster there: FP32 us per step, 512-thread LDS, best register and
+// column kernel: 80 x 70 p5 9.2, 13.4, 7.3; 150 x 102 p7 17.7, 23.3, 11.4;
+// 170 x 163 p8 35.1, 41.1, 21.0.
+// FP64: two passes, after trials of the first candidate that are not counted:
+// in a single one the first candidates run on a GPU that has not reached its
+// clocks and lose to others that are a few percent slower.
+template <typename Select, typename Trial>
+int tune(int p, int mode, int schedule, long nodes, const std::vector<int> &built, int reps, int current,
+         Select select, Trial trial, double *best_ms) {
+  const int half = (reps + 1) / 2;
+  std::vector<int> cands;
+  int best = -1;
+  if (mode == SE2W_FP64) {
+    for (int v : built)
+      if (tuning_candidate(p, schedule, nodes, v)) cands.push_back(v);
+    if (cands.size() > 1) fastest_of({cands[0]}, 1, half, select, trial, best_ms);
+    best = fastest_of(cands, 2, half, select, trial, best_ms);
+  } else {
+    for (int v : built)
+      if (!is_col_variant(v)) cands.push_back(v);
+    best = fastest_of(cands, 1, reps, select, trial, best_ms);
+    if (is_reg_variant(best)) {
+      cands = {best};
+      for (int v : built)
+        if (is_col_variant(v)) cands.push_back(v);
+      const int faster = cands.size() > 1 ? fastest_of(cands, 2, half, select, trial, best_ms) : -1;
+      if (faster >= 0) best = faster;
+    }
+  }
+  return best < 0 ? current : best;
 }
 
 void reg_shape(int variant, int &tex, int &tey) {
@@ -1400,8 +1462,8 @@ int se2w_set_kernel(se2w_ctx *c, int32_t variant) {
 
 int se2w_kernel_count(void) { return kNumVariants; }
 
-// Autotuner: times every variant built for the context's (p, precision,
-// schedule) on the context's own mesh and keeps the fastest.  The state is
+// Autotuner: times the variants that tune() chooses from on the context's own
+// mesh and keeps the fastest.  The state is
 // snapshotted and restored around the trials, so tuning does not perturb the
 // simulation.  Choices are cached per (p, precision, schedule, size bucket)
 // for the life of the process.
@@ -1490,36 +1552,21 @@ int se2w_autotune(se2w_ctx *c, int32_t steps, int32_t reps, int32_t *best_varian
     cands.push_back(SE2W_KERNEL_MFMA);
     cands.push_back(SE2W_KERNEL_LINE);
   }
-  cands.erase(std::remove_if(cands.begin(), cands.end(),
-                             [&](int v) { return !tuning_candidate(c->p, c->mode, c->schedule, (long)c->nx * c->ny, v); }),
-              cands.end());
   Snapshot sn;
   if (int ierr = snapshot_take(c, sn)) return ierr;
   const int variant0 = c->variant;
   std::vector<double> zeros((size_t)steps * std::max(c->ns, 1), 0.0);
-  int best = variant0;
   double best_t = 1e300;
   const bool prof0 = c->profiling;
   c->profiling = true;
-  // Two rounds over the candidates, each with half the trials: in
-  // one round the first candidates run on a GPU that has not reached its
-  // clocks and lose to others that are a few percent slower.
-  const int half = (reps + 1) / 2;
-  std::map<int, std::vector<double>> times;
-  for (int round = 0; round < 2; round++)
-    for (int v : cands) {
-      if (se2w_set_kernel(c, v)) continue;
-      int ierr = SE2W_OK;
-      for (int r = 0; r < half + 1 && !ierr; r++) {  // first repetition is a warm-up
-        ierr = se2w_run(c, steps, 1.0e-30, zeros.data());
-        if (!ierr && r > 0 && (round > 0 || v != cands[0])) times[v].push_back(c->kern_ms[0] + c->kern_ms[1]);
-      }
-    }
-  for (auto &[v, t] : times) {
-    std::sort(t.begin(), t.end());
-    const double med = t[t.size() / 2];
-    if (med < best_t) { best_t = med; best = v; }
-  }
+  const int best = tune(
+      c->p, c->mode, c->schedule, (long)c->nx * c->ny, cands, reps, variant0, [&](int v) { return se2w_set_kernel(c, v); },
+      [&](double *ms) {
+        const int ierr = se2w_run(c, steps, 1.0e-30, zeros.data());
+        *ms = c->kern_ms[0] + c->kern_ms[1];
+        return ierr;
+      },
+      &best_t);
   c->profiling = prof0;
   if (int ierr = snapshot_restore(c, sn)) return ierr;
   int ierr = se2w_set_kernel(c, best);
@@ -1799,7 +1846,7 @@ int se2w_ensemble_autotune(se2w_ensemble *e, int32_t steps, int32_t reps, int32_
   long nodes = 0;
   for (const se2w_ctx *c : e->members) nodes += (long)c->nx * c->ny;
   for (int v = 0; v < kNumVariants; v++)
-    if (ens_variant_built(e, v) && tuning_candidate(e->p, e->mode, SE2W_SCHED_FUSED, nodes, v)) cands.push_back(v);
+    if (ens_variant_built(e, v)) cands.push_back(v);
   const size_t n = e->members.size();
   std::vector<Snapshot> sn(n);
   for (size_t i = 0; i < n; i++) {
@@ -1818,21 +1865,15 @@ int se2w_ensemble_autotune(se2w_ensemble *e, int32_t steps, int32_t reps, int32_
   const int variant0 = e->variant;
   const bool graph0 = e->use_graph;
   e->use_graph = false;
-  int best = variant0;
   double best_t = 1e300;
-  for (int v : cands) {
-    if (ens_set_variant(e, v)) continue;
-    std::vector<double> t;
-    int ierr = SE2W_OK;
-    for (int r = 0; r < reps + 1 && !ierr; r++) {  // first repetition is a warm-up
-      ierr = ens_run(e, steps, dts.data(), psi.data());
-      if (!ierr && r > 0) t.push_back(e->step_ms);
-    }
-    if (ierr || t.empty()) continue;
-    std::sort(t.begin(), t.end());
-    const double med = t[t.size() / 2];
-    if (med < best_t) { best_t = med; best = v; }
-  }
+  const int best = tune(
+      e->p, e->mode, SE2W_SCHED_FUSED, nodes, cands, reps, variant0, [&](int v) { return ens_set_variant(e, v); },
+      [&](double *ms) {
+        const int ierr = ens_run(e, steps, dts.data(), psi.data());
+        *ms = e->step_ms;
+        return ierr;
+      },
+      &best_t);
   e->use_graph = graph0;
   int ierr = SE2W_OK;
   for (size_t i = 0; i < n; i++) {

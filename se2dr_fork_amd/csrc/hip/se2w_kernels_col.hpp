@@ -27,11 +27,15 @@
 //
 // Every sum runs over the same terms in the same order, with the same
 // roundings, as in reg64_body / reg_body, so the results have the same bits
-// (FP64: those of the reference's loop).  One exception: the diagonal terms
-// of a row sum (the node or point of the lane's own column) are added through
-// a multiply-add with a factor 1 or 0, which differs from adding them on that
-// one lane only when the term is infinite, that is after an overflow of the
-// displacement.
+// (FP64: those of the reference's loop).  In FP64 the diagonal term of a row
+// sum (the node or point of the lane's own column) is added by a multiply-add
+// with a factor 1 or 0, one instruction of the three of a term.  The factor 0
+// makes a NaN of an infinite term, and a NaN of every force that this touches:
+// a wave that finds a NaN among its forces forms them again without the factor
+// (col_force_f64).  Adding the term through a select instead is exact too and
+// takes 2 to 9 % longer (us per step, this form and the select: 300^2 p3 18.3,
+// 19.0, 220^2 p6 39.8, 41.3, 64^2 p7 15.0, 16.4, 256^2 p8 95, 99); under an
+// execution mask of the lane's column it takes 0 to 10 % longer.
 //
 // Tiling: as in the register kernels, a workgroup owns its elements except
 // the left column and the bottom row, which only supply their edge forces;
@@ -84,6 +88,62 @@ __device__ __forceinline__ double lane_value(double v, int t) {
   const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)b, t);
   const int hi = __builtin_amdgcn_readlane((int)(b >> 32), t);
   return __longlong_as_double((long long)hi << 32 | lo);
+}
+
+// FP64 force of the node (i, j) from the displacement of its element, which B
+// holds: the terms, their order and their roundings as in col_body, each
+// stress formed where it is used.  Only for waves with a NaN among their
+// forces, so small and slow: rolled loops, in which no lane uses another's
+// stresses.  A second copy of the unrolled operator makes the first one spill.
+template <int P, typename PRM>
+__device__ double2 col_force_f64(PRM &prm, const double2 *B, const double *dny, double iJ00, double detJ, double lam,
+                                 double mu, int i, int j) {
+#pragma clang fp contract(off)
+  constexpr int NB = P + 1;
+  const double c11 = 2.0 * mu + lam;
+  struct Stress { double xx, xy, yy; };
+  auto stress = [&](int k, int q) {  // at the point (k, q)
+    double e0 = 0.0, e1 = 0.0, e2 = 0.0;
+#pragma unroll 1
+    for (int l = 0; l < NB; l++) {
+      const double dy = dny[q * NB + l];
+      const double2 ul = B[l * NB + k];
+      e1 = e1 + dy * ul.y;
+      if (l != q) {
+        e2 = e2 + dy * ul.x;
+        continue;
+      }
+#pragma unroll 1
+      for (int m = 0; m < NB; m++) {
+        const double dx = iJ00 * prm.D[k * NB + m];
+        const double2 um = B[q * NB + m];
+        e0 = e0 + dx * um.x;
+        e2 = e2 + (m == k ? dy * ul.x + dx * um.y : dx * um.y);
+      }
+    }
+    return Stress{c11 * e0 + lam * e1, mu * e2, lam * e0 + c11 * e1};
+  };
+  double2 f = double2{0.0, 0.0};
+#pragma unroll 1
+  for (int q = 0; q < NB; q++) {
+    const Stress s = stress(i, q);
+    const double dy = dny[q * NB + j];
+    if (q != j) {
+      const double nfac = -(detJ * prm.w2[i * NB + q]);
+      f.x = f.x + nfac * (dy * s.xy);
+      f.y = f.y + nfac * (dy * s.yy);
+      continue;
+    }
+#pragma unroll 1
+    for (int k = 0; k < NB; k++) {
+      const Stress t = stress(k, j);
+      const double nfac = -(detJ * prm.w2[j * NB + k]), dx = iJ00 * prm.D[k * NB + i];
+      const double x = dx * t.xx, y = dx * t.xy;
+      f.x = f.x + nfac * (k == i ? dy * s.xy + x : x);
+      f.y = f.y + nfac * (k == i ? dy * s.yy + y : y);
+    }
+  }
+  return f;
 }
 
 template <int P, int MODE, int WX, int EY, typename PRM>
@@ -250,6 +310,36 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
 #pragma unroll
           for (int j = 0; j < NB; j++)
             if (j != qj) column_term(qj, j, dq, F[j]);
+        }
+      }
+      // Infinite forces of both signs make a NaN of the sum too, which costs
+      // time and changes nothing.
+      R sum = F[P].x + F[P].y;
+      if (ly != 0) {
+#pragma unroll
+        for (int j = 0; j < P; j++) sum = sum + F[j].x + F[j].y;
+      }
+      if (__builtin_expect(__any(__builtin_isnan(sum)), 0)) {  // uniform per wave
+        // Element and column again from the thread's index: held from above
+        // they take registers of the operator (300 x 300 p7: 94 -> 111 us).
+        int l = threadIdx.x;
+        asm volatile("" : "+v"(l));
+        l &= 63;
+        const int le = min(l / NB, EPW - 1), col = min(l - le * NB, P), bx = (wave % WX) * EPW + le;
+        const int x = min(max(ex0 - 1 + bx, 0), prm.mx - 1), el = x + ey * prm.mx;
+        R2 *E = &buf[ly][bx][0];
+        const R hx = R(0.5) * prm.elem_dx[x], hy = R(0.5) * prm.elem_dy[ey];
+        wave_lds_order();
+#pragma unroll 1
+        for (int j = 0; j < NB; j++) E[j * NB + col] = prm.u_in[(long)(ey * P + j) * prm.pitch + x * P + col];
+        wave_lds_order();
+#pragma unroll 1
+        for (int n = ly != 0 ? 0 : P; n < NB; n++) {
+          const R2 f = col_force_f64<P>(prm, E, prm.dny + (long)ey * (NB * NB), R(1) / hx, hx * hy, prm.lambda[el],
+                                        prm.mu[el], col, n);
+#pragma unroll
+          for (int j = 0; j < NB; j++)
+            if (j == n) F[j] = f;
         }
       }
     } else {

@@ -758,3 +758,34 @@ def test_tuning_settles_the_order_of_the_sums_without_the_column_kernel(precisio
     want = gpu_run(sc, precision=precision, nsteps=40, kernel=S.KERNEL_LDS if lds else S.KERNEL_REG)
     for got, ref in zip((rows, u, v, a), want[2:]):
         np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("p", range(2, 9))
+def test_fp64_column_kernel_overflows_as_the_other_kernels_do(p):
+    """A state whose strains, stresses or forces overflow: the column kernel
+    leaves the same infinities and NaNs as the LDS kernel, node by node, in the
+    step of the overflow and after it (a diagonal term of a row sum that is
+    infinite reaches its own point or node only)."""
+    rs = np.random.RandomState(40 + p)
+    for big, stiff in ((1e300, 1.0), (3e302, 1.0), (1e304, 1.0), (1e140, 1e150), (1e150, 1e145)):
+        sc = SC.small(mx=9, my=7, p=p, nt=20, seed=p)
+        res = []
+        k = rs.randint(0, 2 * (9 * p + 1) * (7 * p + 1), 5)
+        for kernel in (S.KERNEL_LDS, S.KERNEL_COL):
+            b = SC.build(sc)
+            ctx = b.solver.ctx
+            lam, mu = (np.full(9 * 7, stiff * x) for x in (3e10, 2e10))
+            ctx.set_cells(lam, mu)
+            ctx.set_kernel(kernel)
+            u = np.zeros(2 * ctx.nnodes)
+            u[k] = big * np.array([1.0, -1.0, 0.5, 1.0, 0.3])
+            ctx.set_state(u, np.zeros_like(u), np.zeros_like(u))
+            out = []
+            for _ in range(3):
+                out.append(b.solver.advance(1, b.dt)[1])
+                out += ctx.get_state()
+            res.append(out)
+            b.solver.close()
+        assert not all(np.isfinite(x).all() for x in res[0])
+        for x, y in zip(*res):
+            np.testing.assert_array_equal(y, x)

@@ -1724,15 +1724,19 @@ int ens_run_mode(se2w_ensemble *e, int nsteps, const double *dt) {
     se2w_ctx *c = e->members[i];
     c->cur ^= ((nsteps - 1) & 1);  // the last step's input: the plain displacement
     close_run(c, dt[i]);
+  }
+  int ierr = SE2W_OK;
+  for (se2w_ctx *c : e->members) {
     if (c->nr == 0) continue;
-    if (int ierr = ensure_stage(c)) return ierr;
+    if ((ierr = ensure_stage(c))) break;
     e->copies[nc++] = CopyItem{(const uint32_t *)c->d_rec, (uint32_t *)c->h_stage,
                                (long)((size_t)nsteps * c->nr * rec_stride(c->p) * real_size(c->mode) / 4)};
-    c->rec_staged = true;
   }
-  launch_copies(e, inputs, nc);
+  if (!ierr) launch_copies(e, inputs, nc);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(e->stream));
+  if (ierr) return ierr;  // no record is staged: each is downloaded when it is asked for
+  for (se2w_ctx *c : e->members) c->rec_staged = c->nr > 0;
   float a = 0.f, b = 0.f;
   HIPCHK(hipEventElapsedTime(&a, e->ev0, e->ev2));
   HIPCHK(hipEventElapsedTime(&b, e->ev1, e->ev2));

@@ -1,0 +1,69 @@
+"""Failure paths of the GPU library's host code, on the CPU: allocations that
+fail in the middle of a call.  Each case runs in a process of its own in which
+tests/fake_hip/fake_hip.c stands in for the HIP runtime (nothing is launched,
+a download fills its destination with a byte)."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+PRELUDE = """
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_live.restype = ctypes.c_size_t
+fake.fake_fail_next.argtypes = [ctypes.c_int, ctypes.c_size_t]
+DEVICE, PINNED = 0, 1
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+import se2dr_fork_amd as S
+from se2dr_fork_amd import scenarios as SC
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    if shutil.which("gcc") is None:
+        pytest.skip("gcc is not installed")
+    if not os.path.exists(os.path.join(ROOT, "se2dr_fork_amd", "lib", "libse2w_hip.so")):
+        pytest.skip("libse2w_hip.so is not built")
+    so = str(tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so")
+    subprocess.run(["gcc", "-O1", "-Wall", "-Werror", "-fPIC", "-shared", "-o", so,
+                    os.path.join(ROOT, "tests", "fake_hip", "fake_hip.c")], check=True)
+
+    def run(body):
+        env = dict(os.environ, SE2W_AUTOTUNE="0", OMP_NUM_THREADS="2")
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body, so, ROOT], capture_output=True, text=True, timeout=120,
+                           env=env)
+        assert r.returncode == 0 and "case ok" in r.stdout, r.stdout[-2000:] + r.stderr[-4000:]
+
+    return run
+
+
+def test_ensemble_rows_after_a_record_buffer_that_could_not_grow(fake):
+    """The second member's pinned record buffer cannot grow: the run fails,
+    and the first member's rows are then downloaded, not read from a buffer
+    that no copy of this run has filled."""
+    fake("""
+builts = [SC.build(SC.small(mx=6, my=5, p=3, nt=20, seed=i, nrec=n)) for i, n in ((1, 2), (2, 5))]
+ens = S.Ensemble([b.solver for b in builts])
+dts = [b.dt for b in builts]
+ens.advance(4, dts)
+fake.fake_fail_next(PINNED, 6 * 5 * (6 + 2 * 4) * 8)
+try:
+    ens.advance(6, dts)
+    raise SystemExit("the run did not fail")
+except S.Se2wError as e:
+    assert "hipHostMalloc" in str(e), e
+fake.fake_fill(0x3f)
+n = fake.fake_downloads()
+rows = builts[0].solver.ctx.receivers()
+assert fake.fake_downloads() == n + 1
+assert rows.shape == (6, 2, 7) and (rows[..., :6] == np.frombuffer(b"\\x3f" * 8)[0]).all()
+rows = builts[1].solver.ctx.receivers()
+assert fake.fake_downloads() == n + 2
+print("case ok")
+""")

@@ -644,16 +644,15 @@ int stage_batch(se2w_mlp *m, int n, const float *x, const float *t) {
   return SE2W_OK;
 }
 
-// Squared-error sums of `batches` batches.
+// Squared-error sums of `batches` batches.  A buffer that cannot grow stays:
+// the loss of a gradient is written to it.
 int ensure_parts(se2w_mlp *m, int batches) {
   if (batches <= m->part_batches) return SE2W_OK;
-  if (m->part) hipFree(m->part);
-  m->part = nullptr;
-  m->part_batches = 0;
-  if (hipMalloc(&m->part, sizeof(double) * (size_t)batches * m->nparts) != hipSuccess) {
-    m->part = nullptr;
+  double *part = nullptr;
+  if (hipMalloc(&part, sizeof(double) * (size_t)batches * m->nparts) != hipSuccess)
     return mfail(SE2W_ERR_MEM, "hipMalloc failed");
-  }
+  if (m->part) hipFree(m->part);
+  m->part = part;
   m->part_batches = batches;
   return SE2W_OK;
 }

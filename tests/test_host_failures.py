@@ -67,3 +67,28 @@ rows = builts[1].solver.ctx.receivers()
 assert fake.fake_downloads() == n + 2
 print("case ok")
 """)
+
+
+def test_gradient_buffers_after_a_training_that_could_not_grow_them(fake):
+    """The buffer of the batches' squared errors cannot grow for an epoch: the
+    training fails, and the buffer of one batch, which the loss of a gradient
+    is written to, is still there."""
+    fake("""
+net = S.Mlp([66, 64, 192], batch=64, seed=1)
+x, t = np.zeros((4 * 64, 66), np.float32), np.zeros((4 * 64, 192), np.float32)
+net.set_data(x, t)
+parts = (64 // 16) * (192 // 16)  # workgroups of the last product
+before = fake.fake_live(DEVICE)
+fake.fake_fail_next(DEVICE, 8 * 4 * parts)
+try:
+    net.train(1)
+    raise SystemExit("the training did not fail")
+except S.Se2wError as e:
+    assert "hipMalloc" in str(e), e
+assert fake.fake_live(DEVICE) == before
+net.gradient(x[:64], t[:64])
+net.train(1)
+net.close()
+assert fake.fake_live(DEVICE) == 0 and fake.fake_live(PINNED) == 0
+print("case ok")
+""")

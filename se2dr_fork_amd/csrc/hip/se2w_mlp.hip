@@ -14,6 +14,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
+#include <new>
 #include <vector>
 
 #include "se2w.h"
@@ -809,34 +811,42 @@ int se2w_mlp_param_count(se2w_mlp *m, int64_t *count) {
   return SE2W_OK;
 }
 
-// Copy between the packed host layout and the padded device weights.  Rows
-// are padded only where the input width is not a multiple of 64 (the first
-// layer): that matrix goes through a padded host copy in one piece, since a
-// 2D copy of pageable memory moves row by row (48 ms for 1024 rows).
+// Copy of a matrix between packed host rows of `in` values and device rows of
+// `pad`.  Padded rows go through a host copy of a few MB at a time: a 2D copy
+// of pageable memory moves row by row (48 ms for 1024 rows).  Packed copies
+// are only queued on the stream.
+static int copy_rows(se2w_mlp *m, float *host, float *dev, int rows, int in, int pad, bool to_host) {
+  const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
+  if (in == pad) {
+    MCHK(hipMemcpyAsync(to_host ? host : dev, to_host ? dev : host, sizeof(float) * (size_t)rows * in, kind, m->stream));
+    return SE2W_OK;
+  }
+  const int block = std::min(rows, std::max(1, (1 << 20) / pad));
+  std::unique_ptr<float[]> buf(new (std::nothrow) float[(size_t)block * pad]());  // the padding is zero
+  if (!buf) return mfail(SE2W_ERR_MEM, "out of host memory");
+  for (int r0 = 0; r0 < rows; r0 += block) {
+    const int n = std::min(block, rows - r0);
+    float *d = dev + (size_t)r0 * pad, *h = host + (size_t)r0 * in;
+    if (!to_host)
+      for (int r = 0; r < n; r++) memcpy(&buf[(size_t)r * pad], h + (size_t)r * in, sizeof(float) * in);
+    MCHK(hipMemcpyAsync(to_host ? buf.get() : d, to_host ? d : buf.get(), sizeof(float) * (size_t)n * pad, kind, m->stream));
+    MCHK(hipStreamSynchronize(m->stream));
+    if (to_host)
+      for (int r = 0; r < n; r++) memcpy(h + (size_t)r * in, &buf[(size_t)r * pad], sizeof(float) * in);
+  }
+  return SE2W_OK;
+}
+
+// Copy between the packed host layout and the device weights, whose rows are
+// padded only where the input width is not a multiple of 64 (the first layer).
 static int params_copy(se2w_mlp *m, float *host, bool to_host, const std::vector<float *> &dev_w,
                        const std::vector<float *> &dev_b) {
-  std::vector<float> padded;
-  const hipMemcpyKind kind = to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice;
-  auto copy = [&](float *h, float *d, size_t n) {
-    return hipMemcpyAsync(to_host ? h : d, to_host ? d : h, sizeof(float) * n, kind, m->stream);
-  };
   size_t off = 0;
   for (int l = 0; l < m->nl; l++) {
     const MlpLayer &Ly = m->L[l];
-    float *w = host + off;
-    if (Ly.in == Ly.in_pad) {
-      MCHK(copy(w, dev_w[l], (size_t)Ly.out * Ly.in));
-    } else {
-      padded.assign((size_t)Ly.out * Ly.in_pad, 0.f);
-      if (!to_host)
-        for (int o = 0; o < Ly.out; o++) memcpy(&padded[(size_t)o * Ly.in_pad], w + (size_t)o * Ly.in, sizeof(float) * Ly.in);
-      MCHK(copy(padded.data(), dev_w[l], padded.size()));
-      MCHK(hipStreamSynchronize(m->stream));
-      if (to_host)
-        for (int o = 0; o < Ly.out; o++) memcpy(w + (size_t)o * Ly.in, &padded[(size_t)o * Ly.in_pad], sizeof(float) * Ly.in);
-    }
+    if (int ierr = copy_rows(m, host + off, dev_w[l], Ly.out, Ly.in, Ly.in_pad, to_host)) return ierr;
     off += (size_t)Ly.out * Ly.in;
-    MCHK(copy(host + off, dev_b[l], Ly.out));
+    if (int ierr = copy_rows(m, host + off, dev_b[l], 1, Ly.out, Ly.out, to_host)) return ierr;
     off += Ly.out;
   }
   MCHK(hipStreamSynchronize(m->stream));
@@ -961,9 +971,7 @@ int se2w_mlp_set_data(se2w_mlp *m, int32_t n, const float *x, const float *targe
   m->ndata = 0;
   MCHK(hipMalloc(&m->X, sizeof(float) * (size_t)n * m->in_pad));
   MCHK(hipMalloc(&m->T, sizeof(float) * (size_t)n * m->out));
-  std::vector<float> padded((size_t)n * m->in_pad, 0.f);  // in one piece, as in params_copy
-  for (int r = 0; r < n; r++) memcpy(&padded[(size_t)r * m->in_pad], x + (size_t)r * m->in, sizeof(float) * m->in);
-  MCHK(hipMemcpyAsync(m->X, padded.data(), sizeof(float) * padded.size(), hipMemcpyHostToDevice, m->stream));
+  if (int ierr = copy_rows(m, const_cast<float *>(x), m->X, n, m->in, m->in_pad, false)) return ierr;
   MCHK(hipMemcpyAsync(m->T, target, sizeof(float) * (size_t)n * m->out, hipMemcpyHostToDevice, m->stream));
   MCHK(hipStreamSynchronize(m->stream));
   m->ndata = n;

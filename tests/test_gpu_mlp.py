@@ -143,3 +143,24 @@ def test_a_training_step_is_its_gradient_and_one_adam_step(widths, batch):
     assert loss == pytest.approx(loss_b, rel=1e-6)
     a.close()
     b.close()
+
+
+def test_padded_rows_in_several_blocks():
+    """Weights and training rows whose padded copies pass through the host in
+    more than one block of 2^20 values, the last one not full: parameters come
+    back as they were set, and a trained batch sees its own rows."""
+    widths = [70, 9280, 64]  # first layer: rows of 70 padded to 128, 8192 of 9280 in the first block
+    m = S.Mlp(widths, batch=64, seed=3)
+    p = np.random.default_rng(1).uniform(-0.1, 0.1, m.nparams).astype(np.float32)
+    m.set_params(p)
+    np.testing.assert_array_equal(m.params(), p)
+    m.close()
+    small, n = [70, 64, 64], 8192 + 192
+    rng = np.random.default_rng(2)
+    x, t = rng.standard_normal((n, 70)).astype(np.float32), rng.standard_normal((n, 64)).astype(np.float32)
+    a = S.Mlp(small, batch=n, seed=4)  # one batch of all rows: a row out of place changes the gradient
+    a.set_data(x, t)
+    loss = a.train(1, lr=1e-3, seed=7)[0]
+    y = S.Mlp(small, batch=n, seed=4).forward(x)
+    assert loss == pytest.approx(float(np.mean((y.astype(np.float64) - t) ** 2)), rel=1e-5)
+    a.close()

@@ -92,3 +92,20 @@ net.close()
 assert fake.fake_live(DEVICE) == 0 and fake.fake_live(PINNED) == 0
 print("case ok")
 """)
+
+
+def test_training_data_needs_no_second_copy_in_host_memory(fake):
+    """Rows of one input are padded to 64 on the device; on the way there the
+    host holds a few megabytes of padded rows, not all of them (512 MB)."""
+    fake("""
+import resource
+net = S.Mlp([1, 64, 64], batch=64, seed=1)
+n = 1 << 21
+x, t = np.ones((n, 1), np.float32), np.zeros((n, 64), np.float32)  # t's pages are never touched
+before = resource.getrusage(resource.RUSAGE_SELF).ru_maxrss
+net.set_data(x, t)
+grown = resource.getrusage(resource.RUSAGE_SELF).ru_maxrss - before
+assert grown < 100 << 10, grown  # KB
+net.close()
+print("case ok")
+""")

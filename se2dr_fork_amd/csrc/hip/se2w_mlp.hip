@@ -217,12 +217,12 @@ __global__ void k_gather(const float *X, const int *idx, int B, int in_pad, bf16
 
 // Rows of a forward batch, read in place from pinned host memory (a batch is
 // some tens of KB; its upload by a copy command took longer than the network
-// for one row): rows x[n][in] become the input operand, zero in the padding
-// and in the rows past n.
-__global__ void k_rows(const float *x, int n, int in, int in_pad, bf16 *H0) {
+// for one row): x[n][in] become the rows from row0 of the input operand, zero
+// in the padding and in the rows past n.
+__global__ void k_rows(const float *x, int n, int row0, int in, int in_pad, bf16 *H0) {
   const int r = blockIdx.x;
-  for (int k = threadIdx.x; k < in_pad; k += blockDim.x)
-    H0[op_index(r, k, in_pad)] = (bf16)(r < n && k < in ? x[(long)r * in + k] : 0.f);
+  for (int k = blockIdx.y * blockDim.x + threadIdx.x; k < in_pad; k += gridDim.y * blockDim.x)
+    H0[op_index(row0 + r, k, in_pad)] = (bf16)(r < n && k < in ? x[(long)r * in + k] : 0.f);
 }
 
 // Download of n 16-byte pieces into pinned host memory: queued behind the
@@ -467,10 +467,10 @@ struct se2w_mlp {
   // per-workgroup squared errors of the batches of an epoch, nparts each
   double *part = nullptr;
   int nparts = 0, part_batches = 0;
-  // se2w_mlp_forward's pinned buffers: the input rows of kAhead + 1 batches
-  // and kAhead chunks of chunk_rows() output rows, with the events of each
+  // se2w_mlp_forward's pinned buffers: kAhead + 1 pieces of input rows and
+  // kAhead chunks of output rows, with the events of each
   float *x_host = nullptr, *y_host = nullptr;
-  hipEvent_t y_up[kAhead] = {}, f0[kAhead + 1] = {}, f1[kAhead + 1] = {};
+  hipEvent_t x_read[kAhead + 1] = {}, y_up[kAhead] = {}, f0[kAhead + 1] = {}, f1[kAhead + 1] = {};
   double *loss = nullptr;  // loss of one batch (se2w_mlp_gradient)
   // two permutations (this epoch's and the next one's), device and pinned
   int *perm_dev = nullptr, *perm_host = nullptr;
@@ -664,8 +664,14 @@ int ensure_parts(se2w_mlp *m, int batches) {
 // a product writes at once.
 int chunk_rows(const se2w_mlp *m) { return std::min(m->B, std::max(16, (1 << 18) / m->out)); }
 
+// Input rows of one pinned piece: a batch up to about 1 MB, so that what a
+// network pins does not grow with its batch (pinning 5 x 134 MB took 250 ms).
+int piece_rows(const se2w_mlp *m) { return std::min(m->B, std::max(1, (1 << 18) / m->in)); }
+
 int forward_buffers(se2w_mlp *m) {
   for (hipEvent_t &e : m->y_up)
+    if (!e) MCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  for (hipEvent_t &e : m->x_read)
     if (!e) MCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   for (int s = 0; s <= kAhead; s++) {
     if (!m->f0[s]) MCHK(hipEventCreate(&m->f0[s]));
@@ -673,7 +679,7 @@ int forward_buffers(se2w_mlp *m) {
   }
   // Filled once: the host's first touch of a pinned page costs a fault each,
   // which the first forward would pay.
-  const size_t nx = (size_t)(kAhead + 1) * m->B * m->in, ny = (size_t)kAhead * chunk_rows(m) * m->out;
+  const size_t nx = (size_t)(kAhead + 1) * piece_rows(m) * m->in, ny = (size_t)kAhead * chunk_rows(m) * m->out;
   if (!m->x_host) {
     MCHK(hipHostMalloc((void **)&m->x_host, sizeof(float) * nx, hipHostMallocDefault));
     memset(m->x_host, 0, sizeof(float) * nx);
@@ -891,6 +897,12 @@ int se2w_mlp_forward(se2w_mlp *m, int32_t n, const float *x, float *y) {
   // copies the earlier ones out.
   const int cr = chunk_rows(m), per = (m->B + cr - 1) / cr;  // chunks of a whole batch
   const int nchunks = n / m->B * per + (n % m->B + cr - 1) / cr;
+  const int xr = piece_rows(m);
+  const bool split = xr < m->B;  // batches of several input pieces
+  // workgroups of a row: a piece of long rows has few of them (256 rows of
+  // 16384: 0.55 ms, with one workgroup a row 2.9)
+  const int row_blocks = std::min(64, (m->in_pad + 1023) / 1024);
+  long piece = 0;
   auto enqueue = [&](int c) -> int {
     const int b = c / per, s = b % (kAhead + 1), r0 = b * m->B, k = std::min(m->B, n - r0);
     const int c0 = (c % per) * cr, rows = std::min(cr, k - c0);
@@ -898,11 +910,19 @@ int se2w_mlp_forward(se2w_mlp *m, int32_t n, const float *x, float *y) {
     // few rows are written to the pinned chunk by the last product itself
     const bool direct = k <= 16;
     if (c % per == 0) {
-      float *xh = m->x_host + (size_t)s * m->B * m->in;
-      memcpy(xh, x + (size_t)r0 * m->in, sizeof(float) * (size_t)k * m->in);
       const int M = k <= 16 ? 16 : k <= 32 ? 32 : round_up(k, 64);
-      MCHK(hipEventRecord(m->f0[s], m->stream));
-      hipLaunchKernelGGL(k_rows, dim3(M), dim3(128), 0, m->stream, (const float *)xh, k, m->in, m->in_pad, m->H0);
+      for (int p0 = 0; p0 < k; p0 += xr, piece++) {
+        const int slot_x = piece % (kAhead + 1), rows_x = std::min(xr, k - p0);
+        const bool last = p0 + xr >= k;
+        // Whole batches: the chunks of the batch that had the slot are copied out.
+        if (split && piece > kAhead) MCHK(hipEventSynchronize(m->x_read[slot_x]));
+        float *xh = m->x_host + (size_t)slot_x * xr * m->in;
+        memcpy(xh, x + (size_t)(r0 + p0) * m->in, sizeof(float) * (size_t)rows_x * m->in);
+        if (last) MCHK(hipEventRecord(m->f0[s], m->stream));
+        hipLaunchKernelGGL(k_rows, dim3(last ? M - p0 : rows_x, row_blocks), dim3(128), 0, m->stream, (const float *)xh, rows_x, p0,
+                           m->in, m->in_pad, m->H0);
+        if (split) MCHK(hipEventRecord(m->x_read[slot_x], m->stream));
+      }
       if (int ierr = forward(m, M, nullptr, direct ? slot : m->Y)) return ierr;
       MCHK(hipEventRecord(m->f1[s], m->stream));
     }
@@ -1076,6 +1096,8 @@ int se2w_mlp_destroy(se2w_mlp *m) {
   if (m->x_host) hipHostFree(m->x_host);
   if (m->y_host) hipHostFree(m->y_host);
   for (hipEvent_t e : m->y_up)
+    if (e) hipEventDestroy(e);
+  for (hipEvent_t e : m->x_read)
     if (e) hipEventDestroy(e);
   for (int s = 0; s <= kAhead; s++) {
     if (m->f0[s]) hipEventDestroy(m->f0[s]);

@@ -164,3 +164,18 @@ def test_padded_rows_in_several_blocks():
     y = S.Mlp(small, batch=n, seed=4).forward(x)
     assert loss == pytest.approx(float(np.mean((y.astype(np.float64) - t) ** 2)), rel=1e-5)
     a.close()
+
+
+@pytest.mark.parametrize("win,rows", [(16384, [1, 15, 16, 17, 48, 63, 64, 65, 7 * 64 + 5]), (300000, [1, 2, 6, 70])])
+def test_forward_inputs_in_several_pieces(win, rows):
+    """Wide inputs, of which a batch passes through the pinned buffer in pieces
+    (16 rows, 1 row), on both sides of pieces and batches and round the ring
+    of five pieces: every row as in a call of its own."""
+    m = S.Mlp([win, 64, 64], batch=64, seed=5)
+    x = np.random.default_rng(3).standard_normal((max(rows), win)).astype(np.float32)
+    one = np.concatenate([m.forward(r) for r in x])
+    y0, _ = M.forward(m.params(), [win, 64, 64], x[:16])
+    assert rel_l2(one[:16], y0) < 5e-3
+    for n in rows:
+        np.testing.assert_array_equal(m.forward(x[:n]), one[:n])
+    m.close()

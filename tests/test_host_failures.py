@@ -109,3 +109,21 @@ assert grown < 100 << 10, grown  # KB
 net.close()
 print("case ok")
 """)
+
+
+def test_a_network_pins_a_bounded_amount_of_host_memory(fake):
+    """Five pieces of input rows and four chunks of output rows, about 1 MB
+    each, whatever the width and the batch (5 x 134 MB of inputs here), and
+    more only for rows that are longer than that."""
+    fake("""
+net = S.Mlp([8192, 64, 64], batch=4096, seed=1)
+assert fake.fake_live(PINNED) <= 9 << 20, fake.fake_live(PINNED)
+net.forward(np.zeros((3 * 4096 + 5, 8192), np.float32))
+assert fake.fake_live(PINNED) <= 9 << 20, fake.fake_live(PINNED)
+net.close()
+net = S.Mlp([1 << 19, 64], batch=64, seed=1)
+assert fake.fake_live(PINNED) <= (5 * 2 << 20) + (4 << 20), fake.fake_live(PINNED)
+net.close()
+assert fake.fake_live(PINNED) == 0
+print("case ok")
+""")

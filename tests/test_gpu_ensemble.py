@@ -196,3 +196,14 @@ def test_ensemble_argument_errors():
     with pytest.raises(S.Se2wError):
         e.set_kernel(99)
     e.close()
+
+
+@pytest.mark.parametrize("members", [1, 2])
+def test_few_members_with_long_records(members):
+    """Records longer than one sweep of the copy's workgroups (128 x 256
+    words over the members), not a multiple of it."""
+    scs = [SC.small(mx=4, my=3, p=3, seed=700 + i, nt=301, nrec=29) for i in range(members)]
+    builts, ens = ensemble(scs, S.FP32)
+    got = ens_runs(builts, ens, 301)
+    assert_same(got, single_runs(scs, S.FP32, 301, kernel=ens.kernel()))
+    ens.close()

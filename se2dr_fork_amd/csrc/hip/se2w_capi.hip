@@ -314,9 +314,12 @@ bool col_variant_built(int p, int mode, int variant, int schedule) {
 // that are the fastest on some mesh.  The LDS kernels are behind from p = 2 on
 // and the register kernels from p = 5 on (the column kernel is 1.4 to 3 times
 // as fast from 24 x 24 elements to 389 x 389).  Below, the column kernel leads
-// up to a million nodes (256 x 256 p4: 22.6 against 26.1 us) and trails on
-// large meshes (800 x 800 p4: 211 against 189 us), where a short trial can
-// mistake it for the faster one: two million is the line.
+// on small meshes and trails on large ones, where a short trial can mistake it
+// for the faster one: two million nodes is the line (us per step, best register
+// and column kernel: p = 4 250 x 250 25.8, 22.5, 354 x 354 40.3, 38.6, 433 x 433
+// 55.3, 58.3, 707 x 707 150, 168; p = 3 333 x 333 22.5, 20.0, 577 x 577 51.4,
+// 49.0, 667 x 667 67.3, 68.0, 943 x 943 145, 157; p = 2 354 x 354 12.2, 12.2,
+// 612 x 612 24.4, 28.5).
 bool tuning_candidate(int p, int schedule, long nodes, int variant) {
   if (p < 2 || schedule != SE2W_SCHED_FUSED) return true;
   if (is_reg64_variant(variant)) return p < 5;
@@ -1469,7 +1472,7 @@ int se2w_kernel_count(void) { return kNumVariants; }
 // for the life of the process.
 namespace {
 std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int, int, int>, int> g_tune_cache;
+std::map<std::tuple<int, int, int, int, int, bool>, int> g_tune_cache;
 int size_bucket(int n) {
   int b = 0;
   while (n > 1) { n >>= 1; b++; }
@@ -1527,7 +1530,9 @@ int se2w_autotune(se2w_ctx *c, int32_t steps, int32_t reps, int32_t *best_varian
   if (!c || steps < 1 || reps < 1) return fail(SE2W_ERR_ARG, "bad autotune arguments");
   if (!c->have_tables || !c->have_cells || !c->have_mass) return fail(SE2W_ERR_STATE, "set tables, cells and mass first");
   HIPCHK(hipSetDevice(c->device));
-  const auto key = std::make_tuple(c->p, c->mode, c->schedule, size_bucket(c->mx), size_bucket(c->my));
+  // the candidates of an FP64 mesh depend on its nodes beside its size class
+  const bool col = c->mode != SE2W_FP64 || tuning_candidate(c->p, c->schedule, (long)c->nx * c->ny, SE2W_KERNEL_COL);
+  const auto key = std::make_tuple(c->p, c->mode, c->schedule, size_bucket(c->mx), size_bucket(c->my), col);
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tune_cache.find(key);

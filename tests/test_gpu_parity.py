@@ -789,3 +789,16 @@ def test_fp64_column_kernel_overflows_as_the_other_kernels_do(p):
         assert not all(np.isfinite(x).all() for x in res[0])
         for x, y in zip(*res):
             np.testing.assert_array_equal(y, x)
+
+
+def test_tuning_does_not_carry_the_column_kernel_past_its_line():
+    """FP64 below p = 5: the column kernel is a candidate up to two million
+    nodes.  Two meshes of one size class on both sides of that line: the
+    larger one is not given what the smaller one was tuned to."""
+    for mx in (260, 500):  # 1.1 and 4.0 million nodes; 256 <= mx < 512
+        sc = SC.small(mx=mx, my=mx, p=4, nt=2)
+        b = SC.build(sc)
+        k = b.solver.ctx.kernel()
+        b.solver.close()
+        assert k in range(S.KERNEL_REG64, S.KERNEL_COL + 1)
+    assert k < S.KERNEL_COL, k

@@ -744,11 +744,16 @@ int se2w_create(const se2w_desc *desc, se2w_ctx **out) {
   c->schedule = desc->schedule;
   c->device = desc->device;
   // Untuned contexts (small meshes, which a trial run would cost more than it
-  // saves): in FP64 the column kernel from p = 3 up, whose waves a small mesh
-  // needs (24 x 24 p4: 9.2 us a step against 21 for the first register
-  // schedule, 24 x 24 p6 15 against 47, 16 x 16 p8 16 against 78; at p = 2 the
-  // two are level), beyond the few elements of a single register-kernel tile.
-  const bool col = c->mode == SE2W_FP64 && c->p >= 3 && (long)c->mx * c->my > 32 &&
+  // saves, and callers that do not tune): in FP64 the column kernel from p = 3
+  // up, whose waves a small mesh needs (us per step, first register schedule and
+  // column kernel: 6 x 6 p3 9.7, 7.9, p4 13.4, 10.1, p6 29.3, 14.8, p8 57, 18;
+  // 16 x 16 p8 78, 17; at p = 2 the two are level up to a million nodes and the
+  // column kernel trails above).  At p = 4 it trails from five million nodes on
+  // (559 x 559 102.8, 103.8, 612 x 612 120, 126; p = 3 leads at every size, 1886 x
+  // 1886 615, 609).  Up to 32 elements the register kernel stays the default (a
+  // test pins it for 6 x 5), not for its time: the column kernel leads there too
+  // (6 x 5 p4 13.9, 10.8, p8 59, 20).
+  const bool col = c->mode == SE2W_FP64 && c->p >= 3 && (long)c->mx * c->my > 32 && (c->p != 4 || nx * ny < 5000000) &&
                    col_variant_built(c->p, c->mode, SE2W_KERNEL_COL, c->schedule);
   c->variant = col ? SE2W_KERNEL_COL
                : reg_available(c->p, c->mode) && reg_variant_built(c->p, SE2W_KERNEL_REG, c->schedule)

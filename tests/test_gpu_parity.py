@@ -802,3 +802,21 @@ def test_tuning_does_not_carry_the_column_kernel_past_its_line():
         b.solver.close()
         assert k in range(S.KERNEL_REG64, S.KERNEL_COL + 1)
     assert k < S.KERNEL_COL, k
+
+
+def test_fp64_default_kernel_on_both_sides_of_its_lines():
+    """An untuned FP64 context runs the column kernel from p = 3 up and from
+    33 elements on, at p = 4 up to five million nodes; the first register
+    schedule of its degree elsewhere."""
+    def kernel(mx, my, p):
+        c = S.Context(mx, my, p, precision=S.FP64)
+        k = c.kernel()
+        c.close()
+        return k
+
+    for p in range(2, 9):
+        reg = S.KERNEL_REG64 + 7 if p == 8 else S.KERNEL_REG64
+        assert kernel(8, 4, p) == reg and kernel(32, 1, p) == reg
+        assert kernel(11, 3, p) == (reg if p == 2 else S.KERNEL_COL)
+    assert kernel(500, 500, 4) == S.KERNEL_COL and kernel(600, 600, 4) == S.KERNEL_REG64
+    assert kernel(1000, 1000, 3) == S.KERNEL_COL

@@ -95,9 +95,9 @@ __device__ __forceinline__ double lane_value(double v, int t) {
 // stress formed where it is used.  Only for waves with a NaN among their
 // forces, so small and slow: rolled loops, in which no lane uses another's
 // stresses.  A second copy of the unrolled operator makes the first one spill.
-template <int P, typename PRM>
-__device__ double2 col_force_f64(PRM &prm, const double2 *B, const double *dny, double iJ00, double detJ, double lam,
-                                 double mu, int i, int j) {
+template <int P>
+__device__ double2 col_force_f64(const double2 *B, const double *D, const double *w2, const double *dny, double iJ00,
+                                 double detJ, double lam, double mu, int i, int j) {
 #pragma clang fp contract(off)
   constexpr int NB = P + 1;
   const double c11 = 2.0 * mu + lam;
@@ -115,7 +115,7 @@ __device__ double2 col_force_f64(PRM &prm, const double2 *B, const double *dny, 
       }
 #pragma unroll 1
       for (int m = 0; m < NB; m++) {
-        const double dx = iJ00 * prm.D[k * NB + m];
+        const double dx = iJ00 * D[k * NB + m];
         const double2 um = B[q * NB + m];
         e0 = e0 + dx * um.x;
         e2 = e2 + (m == k ? dy * ul.x + dx * um.y : dx * um.y);
@@ -129,7 +129,7 @@ __device__ double2 col_force_f64(PRM &prm, const double2 *B, const double *dny, 
     const Stress s = stress(i, q);
     const double dy = dny[q * NB + j];
     if (q != j) {
-      const double nfac = -(detJ * prm.w2[i * NB + q]);
+      const double nfac = -(detJ * w2[i * NB + q]);
       f.x = f.x + nfac * (dy * s.xy);
       f.y = f.y + nfac * (dy * s.yy);
       continue;
@@ -137,7 +137,7 @@ __device__ double2 col_force_f64(PRM &prm, const double2 *B, const double *dny, 
 #pragma unroll 1
     for (int k = 0; k < NB; k++) {
       const Stress t = stress(k, j);
-      const double nfac = -(detJ * prm.w2[j * NB + k]), dx = iJ00 * prm.D[k * NB + i];
+      const double nfac = -(detJ * w2[j * NB + k]), dx = iJ00 * D[k * NB + i];
       const double x = dx * t.xx, y = dx * t.xy;
       f.x = f.x + nfac * (k == i ? dy * s.xy + x : x);
       f.y = f.y + nfac * (k == i ? dy * s.yy + y : y);
@@ -312,14 +312,14 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
             if (j != qj) column_term(qj, j, dq, F[j]);
         }
       }
-      // Infinite forces of both signs make a NaN of the sum too, which costs
-      // time and changes nothing.
-      R sum = F[P].x + F[P].y;
+      // Infinite forces of both signs make a NaN of a sum too, which costs time
+      // and changes nothing.
+      R2 sum = F[P];
       if (ly != 0) {
 #pragma unroll
-        for (int j = 0; j < P; j++) sum = sum + F[j].x + F[j].y;
+        for (int j = 0; j < P; j++) sum = R2{sum.x + F[j].x, sum.y + F[j].y};
       }
-      if (__builtin_expect(__any(__builtin_isnan(sum)), 0)) {  // uniform per wave
+      if (__builtin_expect(__any(__builtin_isunordered(sum.x, sum.y)), 0)) {  // uniform per wave
         // Element and column again from the thread's index: held from above
         // they take registers of the operator (300 x 300 p7: 94 -> 111 us).
         int l = threadIdx.x;
@@ -329,14 +329,15 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
         const int x = min(max(ex0 - 1 + bx, 0), prm.mx - 1), el = x + ey * prm.mx;
         R2 *E = &buf[ly][bx][0];
         const R hx = R(0.5) * prm.elem_dx[x], hy = R(0.5) * prm.elem_dy[ey];
+        const R *tD = prm.D, *tw = prm.w2, *tdny = prm.dny + (long)ey * (NB * NB);
+        asm volatile("" : "+v"(tD), "+v"(tw), "+v"(tdny));  // vector registers are free here, scalar ones are not
         wave_lds_order();
 #pragma unroll 1
         for (int j = 0; j < NB; j++) E[j * NB + col] = prm.u_in[(long)(ey * P + j) * prm.pitch + x * P + col];
         wave_lds_order();
 #pragma unroll 1
         for (int n = ly != 0 ? 0 : P; n < NB; n++) {
-          const R2 f = col_force_f64<P>(prm, E, prm.dny + (long)ey * (NB * NB), R(1) / hx, hx * hy, prm.lambda[el],
-                                        prm.mu[el], col, n);
+          const R2 f = col_force_f64<P>(E, tD, tw, tdny, R(1) / hx, hx * hy, prm.lambda[el], prm.mu[el], col, n);
 #pragma unroll
           for (int j = 0; j < NB; j++)
             if (j == n) F[j] = f;
@@ -451,7 +452,9 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
   // With sources and receivers: a lane holds one list entry (64 at a time) and
   // every lane tests its node against each in turn, so the lists cost no memory
   // latency per node (36 elements at p = 8 with 8 receivers: 29 -> 24 us a
-  // step).  The loops are uniform and every lane takes part in them.
+  // step).  The loops are uniform and every lane takes part in them; an entry is
+  // read from its lane before the branch on the node, in which that lane may be
+  // idle and its registers are not kept.
   // The lane's entries of the tile's source and receiver lists, with the node
   // coordinates of their element's first node.
   struct ListItem { int id, x, y, gll; };
@@ -488,10 +491,10 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
       if (tl.s1 - tl.s0 > 64) src = source(t0);
       const int n = min(64, tl.s1 - t0);
       for (int t = 0; t < n; t++) {
-        const int li = gx - lane_value(src.x, t), lj = gy0 + j - lane_value(src.y, t);
+        const int li = gx - lane_value(src.x, t), lj = gy0 + j - lane_value(src.y, t), id = lane_value(src.id, t);
+        const R ps = lane_value(psi, t);
         if (node && li >= 0 && li <= P && lj >= 0 && lj <= P) {
-          const R ps = lane_value(psi, t);
-          const long k = ((long)lane_value(src.id, t) * NB * NB + li + lj * NB) * 2;
+          const long k = ((long)id * NB * NB + li + lj * NB) * 2;
           sum.x = sum.x + ps * prm.src_vals[k];
           sum.y = sum.y + ps * prm.src_vals[k + 1];
           hit = true;
@@ -515,12 +518,12 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
       const int n = min(64, tl.r1 - t0);
       for (int t = 0; t < n; t++) {
         const int li = gx - lane_value(rec.x, t), lj = gy0 + j - lane_value(rec.y, t), g = lane_value(rec.gll, t);
-        const int gi = g % NB, gj = g / NB;
+        const int id = lane_value(rec.id, t), gi = g % NB, gj = g / NB;
         const bool on_column = li == gi && lj >= 0 && lj <= P, on_row = lj == gj && li >= 0 && li <= P;
         if (node && (on_column || on_row)) {
           R2 v, a;
           corrected(v, a);
-          R *o = prm.rec + ((long)step * prm.nr + lane_value(rec.id, t)) * rec_stride(P);
+          R *o = prm.rec + ((long)step * prm.nr + id) * rec_stride(P);
           if (on_column) o[6 + lj] = v.x;
           if (on_row) o[6 + NB + li] = v.y;
           if (on_column && on_row) {
@@ -533,11 +536,11 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
       const ListItem er = list_item(prm.tile_erec_idx, prm.erec_elem, t0, tl.q1);
       const int n = min(64, tl.q1 - t0);
       for (int t = 0; t < n; t++) {
-        const int li = gx - lane_value(er.x, t), lj = gy0 + j - lane_value(er.y, t);
+        const int li = gx - lane_value(er.x, t), lj = gy0 + j - lane_value(er.y, t), id = lane_value(er.id, t);
         if (node && li >= 0 && li <= P && lj >= 0 && lj <= P) {
           R2 v, a;
           corrected(v, a);
-          R *q = prm.erec + (((long)step * prm.ner + lane_value(er.id, t)) * (NB * NB) + li + lj * NB) * 4;
+          R *q = prm.erec + (((long)step * prm.ner + id) * (NB * NB) + li + lj * NB) * 4;
           q[0] = pu[j].x; q[1] = pu[j].y; q[2] = v.x; q[3] = v.y;
         }
       }

@@ -820,3 +820,25 @@ def test_fp64_default_kernel_on_both_sides_of_its_lines():
         assert kernel(11, 3, p) == (reg if p == 2 else S.KERNEL_COL)
     assert kernel(500, 500, 4) == S.KERNEL_COL and kernel(600, 600, 4) == S.KERNEL_REG64
     assert kernel(1000, 1000, 3) == S.KERNEL_COL
+
+
+@pytest.mark.parametrize("precision", [S.FP32, S.FP32_KAHAN])
+@pytest.mark.parametrize("p, mx, my", [(2, 19, 4), (5, 9, 5), (7, 6, 3), (8, 5, 4)])
+def test_fp32_column_kernel_with_long_lists_on_one_tile(precision, p, mx, my):
+    """More than 64 sources, receivers and element receivers on a tile in the
+    FP32 modes: the bits of the register kernel, for every workgroup shape."""
+    hip, _ = S.libraries()
+    sc = SC.small(mx=mx, my=my, p=p, nt=20, seed=17 + p, nsrc=70, nrec=150)
+    xr = np.random.default_rng(p).uniform(100.0, 3900.0, (70, 2))
+    want = None
+    for k in [S.KERNEL_REG if p < 7 else S.KERNEL_REG + 3, *range(S.KERNEL_COL, hip.se2w_kernel_count())]:
+        b = SC.build(sc, precision=precision)
+        b.solver.ctx.set_kernel(k)
+        b.solver.set_uv_receivers([S.ReceiverUV(b.spec, x, interpolate=True) for x in xr])
+        _, rows = b.solver.advance(b.nsteps, b.dt)
+        got = [rows, *b.solver.ctx.get_state(), b.solver.uv_trace(b.nsteps)]
+        b.solver.close()
+        if want is None:
+            want = got
+        for x, y in zip(got, want):
+            np.testing.assert_array_equal(x, y, err_msg=f"variant {k}")

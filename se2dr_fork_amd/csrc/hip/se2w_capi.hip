@@ -1562,6 +1562,16 @@ int se2w_autotune(se2w_ctx *c, int32_t steps, int32_t reps, int32_t *best_varian
     cands.push_back(SE2W_KERNEL_MFMA);
     cands.push_back(SE2W_KERNEL_LINE);
   }
+  if (c->mode == SE2W_FP64) {
+    cands.erase(std::remove_if(cands.begin(), cands.end(),
+                               [&](int v) { return !tuning_candidate(c->p, c->schedule, (long)c->nx * c->ny, v); }),
+                cands.end());
+    if (cands.size() == 1 && !best_ms) {  // nothing to choose, and nobody asks for its time
+      if (int ierr = se2w_set_kernel(c, cands[0])) return ierr;
+      if (best_variant) *best_variant = cands[0];
+      return SE2W_OK;
+    }
+  }
   Snapshot sn;
   if (int ierr = snapshot_take(c, sn)) return ierr;
   const int variant0 = c->variant;

@@ -12,13 +12,14 @@ enum { OK = 0, OUT_OF_MEMORY = 2, MAX = 4096 };
 
 static struct { void *p; size_t n; int pinned; } live[MAX];
 static size_t fail_size[2], next_address = (size_t)1 << 44;
-static int fill_byte, downloads;
+static int fill_byte, downloads, launches;
 static char handle;
 
 /* kind 0: device, 1: pinned host */
 void fake_fail_next(int kind, size_t bytes) { fail_size[kind] = bytes; }
 void fake_fill(int byte) { fill_byte = byte; }
 int fake_downloads(void) { return downloads; }
+int fake_launches(void) { return launches; }
 size_t fake_live(int kind)
 {
   size_t s = 0;
@@ -103,6 +104,7 @@ int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *sh, void **s)
 int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **a, size_t sh, void *s)
 {
   (void)f; (void)g; (void)b; (void)a; (void)sh; (void)s;
+  launches++;
   return OK;
 }
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *f, int t, size_t sh)

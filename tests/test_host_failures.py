@@ -1,5 +1,5 @@
-"""Failure paths of the GPU library's host code, on the CPU: allocations that
-fail in the middle of a call.  Each case runs in a process of its own in which
+"""The GPU library's host code on the CPU, above all its failure paths:
+allocations that fail in the middle of a call.  Each case runs in a process of its own in which
 tests/fake_hip/fake_hip.c stands in for the HIP runtime (nothing is launched,
 a download fills its destination with a byte)."""
 import os
@@ -125,5 +125,24 @@ net = S.Mlp([1 << 19, 64], batch=64, seed=1)
 assert fake.fake_live(PINNED) <= (5 * 2 << 20) + (4 << 20), fake.fake_live(PINNED)
 net.close()
 assert fake.fake_live(PINNED) == 0
+print("case ok")
+""")
+
+
+def test_tuning_with_one_candidate_runs_no_trial(fake):
+    """In FP64 from p = 5 up only the column kernel is left to a tuner: it is
+    set without trials unless the caller asks for its time."""
+    fake("""
+builts = [SC.build(SC.small(mx=mx, my=my, p=p, nt=20)) for mx, my, p in ((7, 6, 6), (7, 6, 4), (20, 17, 6))]
+ctx, ctx4, ctx6 = [b.solver.ctx for b in builts]
+ctx.set_kernel(S.KERNEL_LDS)
+best, n = ctypes.c_int32(), fake.fake_launches()
+assert ctx._hip.se2w_autotune(ctx._handle, 20, 3, ctypes.byref(best), None) == 0
+assert best.value == ctx.kernel() == S.KERNEL_COL
+assert fake.fake_launches() == n
+assert ctx4._hip.se2w_autotune(ctx4._handle, 20, 3, ctypes.byref(best), None) == 0
+assert fake.fake_launches() > n
+n = fake.fake_launches()
+assert ctx6.autotune()[1] > 0 and fake.fake_launches() > n
 print("case ok")
 """)

@@ -207,3 +207,33 @@ def test_few_members_with_long_records(members):
     got = ens_runs(builts, ens, 301)
     assert_same(got, single_runs(scs, S.FP32, 301, kernel=ens.kernel()))
     ens.close()
+
+
+@pytest.mark.parametrize("p", [2, 3, 5, 6, 7, 8])
+def test_fp64_ensemble_column_kernel_bit_identical_to_oracle(oracle, p):
+    """The batched column kernel, members from one element to several tiles."""
+    scs = uneven(p, n=4, seed=800 + p) + [SC.small(mx=1, my=1, p=p, seed=1), SC.small(mx=41, my=8, p=p, seed=2)]
+    builts, ens = ensemble(scs, S.FP64)
+    ens.set_kernel(S.KERNEL_COL)
+    got = ens_runs(builts, ens, 24, chunks=(11, 13))
+    for sc, b, have in zip(scs, builts, got):
+        want = oracle.Problem(sc, dt=b.dt, nt=24).run(max_steps=24)[1:]
+        for x, y in zip(have, want):
+            np.testing.assert_array_equal(x, y)
+    ens.close()
+
+
+@pytest.mark.parametrize("prec", [S.FP32, S.FP32_KAHAN])
+@pytest.mark.parametrize("p", [2, 4, 5, 6, 7, 8])
+def test_fp32_ensemble_column_kernel_equals_single_runs(prec, p):
+    """Both workgroup shapes of the batched column kernel, against the single
+    column kernel and the register kernel; 70 receivers on one member."""
+    scs = uneven(p, n=4, seed=900 + p) + [SC.small(mx=5, my=4, p=p, seed=3, nsrc=3, nrec=70)]
+    reg = S.KERNEL_REG if p < 7 else S.KERNEL_REG + 3
+    want = single_runs(scs, prec, 24, kernel=reg, chunks=(11, 13))
+    for var in (S.KERNEL_COL, S.KERNEL_COL + 1):
+        assert_same(single_runs(scs, prec, 24, kernel=var, chunks=(11, 13)), want)
+        builts, ens = ensemble(scs, prec)
+        ens.set_kernel(var)
+        assert_same(ens_runs(builts, ens, 24, chunks=(11, 13)), want)
+        ens.close()

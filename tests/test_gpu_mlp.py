@@ -179,3 +179,17 @@ def test_forward_inputs_in_several_pieces(win, rows):
     for n in rows:
         np.testing.assert_array_equal(m.forward(x[:n]), one[:n])
     m.close()
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 63, 64, 65, 127, 128, 129, 192, 6 * 128 + 5, 7 * 128 + 70, 13 * 128])
+def test_forward_in_several_chunks_of_several_batches(rows):
+    """Batches of 128 rows whose outputs come down in two chunks of 64, row
+    counts on both sides of chunks and batches and several times round the
+    four output and five input slots: the rows of calls of their own."""
+    m = S.Mlp([66, 64, 4096], batch=128, seed=6)
+    x = np.random.default_rng(4).standard_normal((rows, 66)).astype(np.float32)
+    want = np.concatenate([m.forward(x[r:r + 48]) for r in range(0, rows, 48)])
+    np.testing.assert_array_equal(m.forward(x), want)
+    y0, _ = M.forward(m.params(), [66, 64, 4096], x[-48:])
+    assert rel_l2(want[-len(x[-48:]):], y0) < 5e-3
+    m.close()

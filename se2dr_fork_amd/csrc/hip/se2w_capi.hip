@@ -326,9 +326,12 @@ bool tuning_candidate(int p, int schedule, long nodes, int variant) {
   return is_col_variant(variant) && (p >= 5 || nodes < 2000000);
 }
 
-// The fastest of `cands` by the median of its trials, -1 if none could run:
-// `rounds` passes over the list, in each of them one untimed and n timed
-// trials of every candidate.  A candidate that fails once is out.
+// The fastest of `cands`, -1 if none could run: `rounds` passes over the list,
+// in each of them one untimed and n timed trials of every candidate.  A single
+// pass compares medians; of several passes the shortest trial counts, since in
+// the first one the first candidates run on a GPU that has not reached its
+// clocks and by their median lose to others that are a few percent slower.  A
+// candidate that fails once is out.
 template <typename Select, typename Trial>
 int fastest_of(const std::vector<int> &cands, int rounds, int n, Select select, Trial trial, double *best_ms) {
   std::vector<std::vector<double>> t(cands.size());
@@ -346,8 +349,8 @@ int fastest_of(const std::vector<int> &cands, int rounds, int n, Select select, 
   for (size_t i = 0; i < cands.size(); i++) {
     if (failed[i] || t[i].empty()) continue;
     std::sort(t[i].begin(), t[i].end());
-    const double med = t[i][t[i].size() / 2];
-    if (best < 0 || med < *best_ms) { *best_ms = med; best = cands[i]; }
+    const double ms = t[i][rounds > 1 ? 0 : t[i].size() / 2];
+    if (best < 0 || ms < *best_ms) { *best_ms = ms; best = cands[i]; }
   }
   return best;
 }
@@ -362,9 +365,7 @@ int fastest_of(const std::vector<int> &cands, int rounds, int n, Select select, 
 // would be faster there: FP32 us per step, 512-thread LDS, best register and
 // column kernel: 80 x 70 p5 9.2, 13.4, 7.3; 150 x 102 p7 17.7, 23.3, 11.4;
 // 170 x 163 p8 35.1, 41.1, 21.0.
-// FP64: two passes, after trials of the first candidate that are not counted:
-// in a single one the first candidates run on a GPU that has not reached its
-// clocks and lose to others that are a few percent slower.
+// FP64: all candidates have the same bits, so the fastest in two passes.
 template <typename Select, typename Trial>
 int tune(int p, int mode, int schedule, long nodes, const std::vector<int> &built, int reps, int current,
          Select select, Trial trial, double *best_ms) {
@@ -374,7 +375,6 @@ int tune(int p, int mode, int schedule, long nodes, const std::vector<int> &buil
   if (mode == SE2W_FP64) {
     for (int v : built)
       if (tuning_candidate(p, schedule, nodes, v)) cands.push_back(v);
-    if (cands.size() > 1) fastest_of({cands[0]}, 1, half, select, trial, best_ms);
     best = fastest_of(cands, 2, half, select, trial, best_ms);
   } else {
     for (int v : built)

@@ -12,12 +12,13 @@ enum { OK = 0, OUT_OF_MEMORY = 2, MAX = 4096 };
 
 static struct { void *p; size_t n; int pinned; } live[MAX];
 static size_t fail_size[2], next_address = (size_t)1 << 44;
-static int fill_byte, downloads, launches;
+static int fill_byte, downloads, launches, slow;
 static char handle;
 
 /* kind 0: device, 1: pinned host */
 void fake_fail_next(int kind, size_t bytes) { fail_size[kind] = bytes; }
 void fake_fill(int byte) { fill_byte = byte; }
+void fake_slow(int n) { slow = n; }  /* the next n times between events are twice as long */
 int fake_downloads(void) { return downloads; }
 int fake_launches(void) { return launches; }
 size_t fake_live(int kind)
@@ -78,7 +79,13 @@ int hipEventCreateWithFlags(void **e, unsigned f) { (void)f; *e = &handle; retur
 int hipEventDestroy(void *e) { (void)e; return OK; }
 int hipEventRecord(void *e, void *s) { (void)e; (void)s; return OK; }
 int hipEventSynchronize(void *e) { (void)e; return OK; }
-int hipEventElapsedTime(float *ms, void *a, void *b) { (void)a; (void)b; *ms = 1.0f; return OK; }
+int hipEventElapsedTime(float *ms, void *a, void *b)
+{
+  (void)a; (void)b;
+  *ms = slow > 0 ? 2.0f : 1.0f;
+  slow -= slow > 0;
+  return OK;
+}
 
 int hipStreamBeginCapture(void *s, int m) { (void)s; (void)m; return OK; }
 int hipStreamEndCapture(void *s, void **g) { (void)s; *g = &handle; return OK; }

@@ -146,3 +146,16 @@ n = fake.fake_launches()
 assert ctx6.autotune()[1] > 0 and fake.fake_launches() > n
 print("case ok")
 """)
+
+
+def test_tuning_does_not_charge_the_first_candidate_with_a_cold_gpu(fake):
+    """Kernels of equal time, of which the first is tried while the GPU is
+    still at half its clocks: the first one stays the choice."""
+    fake("""
+b = SC.build(SC.small(mx=7, my=6, p=4, nt=20))
+ctx, best = b.solver.ctx, ctypes.c_int32()
+fake.fake_slow(12)  # two times are taken of each trial run
+assert ctx._hip.se2w_autotune(ctx._handle, 20, 3, ctypes.byref(best), None) == 0
+assert best.value == S.KERNEL_REG64, best.value
+print("case ok")
+""")

@@ -193,12 +193,16 @@ int se2w_set_kernel(se2w_ctx *ctx, int32_t variant);
 int se2w_get_kernel(se2w_ctx *ctx, int32_t *variant);
 int se2w_kernel_count(void);
 
-/* Autotuner (no counterpart in the reference): runs `reps` timed trials of
- * `steps` steps for every element-kernel variant that is the fastest on some
- * mesh at this context's degree, precision and schedule, keeps the fastest (median kernel time) and
- * reports it.  The state u, v, a is restored afterwards; receiver rows of the
- * previous se2w_run are discarded.  The choice is cached per (p, precision,
- * schedule, size bucket) for the rest of the process. */
+/* Autotuner (no counterpart in the reference): runs timed trials of `steps`
+ * steps (`reps` and more of each) for the element-kernel variants that can be
+ * the fastest at this context's degree, precision and schedule, keeps the
+ * fastest and reports it.  In FP64 all variants have the same bits.  In the
+ * FP32 modes the order of the sums is that of the fastest variant other than
+ * the column kernel, which is a candidate only where it sums in that order.
+ * The state u, v, a is restored afterwards; receiver rows of the previous
+ * se2w_run are discarded.  The choice is cached per (p, precision, schedule,
+ * size class) for the rest of the process (best_ms is then -1).  best_ms may
+ * be NULL: with one candidate left no trial is run then. */
 int se2w_autotune(se2w_ctx *ctx, int32_t steps, int32_t reps, int32_t *best_variant, double *best_ms);
 
 /* Tile shape (owned elements per workgroup) used by the step kernels. */
@@ -220,12 +224,11 @@ int se2w_ensemble_create(int32_t n, se2w_ctx *const *members, se2w_ensemble **en
 /* nsteps steps of every member: dt[i] its time step, psi[i] its
  * source-time table [nsteps][ns_i] (may be NULL for members without sources). */
 int se2w_ensemble_run(se2w_ensemble *ens, int32_t nsteps, const double *dt, const double *const *psi);
-/* Kernel variant of the batched step (SE2W_KERNEL_LDS or SE2W_KERNEL_REG + k),
- * applied to every member. */
+/* Kernel variant of the batched step, applied to every member. */
 int se2w_ensemble_set_kernel(se2w_ensemble *ens, int32_t variant);
 int se2w_ensemble_get_kernel(se2w_ensemble *ens, int32_t *variant);
-/* Times every built variant over `steps` batched steps (reps repetitions,
- * state restored afterwards) and keeps the fastest. */
+/* The choice of se2w_autotune over `steps` batched steps of all members
+ * (state restored afterwards; not cached). */
 int se2w_ensemble_autotune(se2w_ensemble *ens, int32_t steps, int32_t reps, int32_t *best_variant, double *best_ms);
 /* on = 1 (default): replay the run's launches from a captured HIP graph;
  * on = 0: launch them one by one. */

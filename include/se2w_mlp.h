@@ -10,7 +10,7 @@
  * seismograms, and the solver (se2w.h) both generates its training data and
  * measures its error.
  *
- * Shapes: widths[0] inputs (any size; padded to a multiple of 32 inside),
+ * Shapes: widths[0] inputs (any size; padded to a multiple of 64 inside),
  * hidden and output widths multiples of 64, batch a multiple of 64.
  * Parameters are exchanged as one FP32 array: for each layer l, W_l
  * [widths[l+1]][widths[l]] row-major, then b_l [widths[l+1]].

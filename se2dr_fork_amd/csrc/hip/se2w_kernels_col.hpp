@@ -549,11 +549,12 @@ __device__ __forceinline__ void col_body(PRM &prm, int tile, int step, int last)
   }
 }
 
-// Minimum waves per SIMD, i.e. the registers per lane: the most that spill at
-// most a few registers, mostly of the update with lists.  FP64 300 x 300 p7
-// takes 94-97 us at three and 100 at two, 512 x 512 p4 74 at four and 77 at
-// three; at p = 8 three waves spill 50 registers (256 x 256: 114 us, 104-107
-// at two), and FP32+Kahan p = 8 10 at four (512 x 512: 254 us, 230 at three).
+// Minimum waves per SIMD, i.e. the registers per lane: the most at which the
+// waves gain more than the spills cost.  FP64 p = 4 and 6 spill 6 registers, p =
+// 7 spills 32 at three (300 x 300: 90-95 us, 100 at two, without spills), 512 x
+// 512 p4 takes 74 us at four and 77 at three; at p = 8 three waves spill 50
+// registers (256 x 256: 114 us, 95-104 at two), and FP32+Kahan p = 8 10 at four
+// (512 x 512: 254 us, 230 at three).
 constexpr int col_waves(int p, int mode) {
   return mode == MODE_F64 ? (p <= 4 ? 4 : p <= 7 ? 3 : 2) : mode == MODE_F32K && p == 8 ? 3 : 4;
 }
